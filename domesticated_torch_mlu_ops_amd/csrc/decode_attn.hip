@@ -43,271 +43,10 @@
 // the partials (max, sum, normalised row) go to a caller-provided workspace and a combine
 // kernel merges them.  A generic kernel (one wavefront per (query token, query head), VALU)
 // serves every other shape, dtype and scale layout.
-#include "tmo_device.h"
+#include "attn_common.h"
 
 namespace tmo {
 namespace {
-
-typedef short bf16x4 __attribute__((ext_vector_type(4)));
-typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLazy = 8.0f;  // log2 headroom of the lazily moved softmax maximum
-constexpr float kLn2 = 0.6931471805599453f;
-
-// Query rows: token s of sequence i is at element i * q_sb + (row0_i + s) * q_ss + hq * q_sh,
-// row0_i = cu[i] with cu_seq_q (q_sb 0 then) and 0 without; out and lse alike.
-struct AttnParams {
-  const void* q;
-  int64_t q_sb, q_ss, q_sh;      // strides (elements); last dim contiguous
-  const int32_t* cu;             // cu_seq_q [B + 1], or null: S tokens per sequence
-  int32_t S;                     // tokens per sequence (at most, with cu)
-  int32_t ncols;                 // S * g query columns per (sequence, KV head)
-  int32_t ncb;                   // column blocks of 16
-  int64_t total_q;               // q rows with cu: rows outside [0, total_q) are skipped
-  const float* sink;             // [Hq] natural-log logits, or null
-  const void* kc;
-  const void* vc;                // caches [NB, Hkv, BS, k_row / v_row] contiguous
-  int64_t k_row, v_row;          // cache row lengths (elements)
-  const void* ks;                // scales: fp32, or bf16 when s_bf16
-  const void* vs;
-  int32_t s_bf16;
-  int32_t smode;                 // 0 plain caches, 1 per token, 2 per channel, 3 per group
-  int64_t ks_sb, ks_sh, vs_sb, vs_sh;  // per-token scale strides (page, head)
-  const int32_t* bt;
-  int64_t max_blocks;
-  const int32_t* lens;
-  const float* alibi;            // [B, Hq] or null
-  int64_t window;                // < 0: unlimited
-  float scale_log2;              // softmax_scale * log2(e)
-  void* out;
-  int64_t o_sb, o_ss, o_sh;
-  float* lse;                    // null when not requested
-  int64_t lse_sb, lse_ss, lse_sh;
-  int32_t B, Hq, Hkv, g, D, Dv, BS;  // D: query / key head size, Dv: value head size
-  int32_t bs_shift;              // log2(BS) when BS is a power of two, else -1
-  int64_t NB;
-  int32_t q_dtype;               // TMO_DTYPE_*: F32 / F16 / BF16, or I8 / F8E4M3 codes (qs)
-  int32_t o_dtype;               // output TMO_DTYPE_* (q's for unquantised q)
-  const void* qs;                // q scales of I8 / F8E4M3 q: fp32, or bf16 when qs_bf16
-  int32_t qs_mode;               // 0 none, 1 per tensor, 2 per (token, head), 3 per channel group
-  int32_t qs_bf16;
-  int64_t qs_sb, qs_ss, qs_sh;   // q scale strides (sequence, token, head), as q's
-  int32_t qs_group;              // mode 3: channels per scale (head_size / scale_num)
-  int64_t bt_heads;              // block-table rows per sequence: 0 ([B, MB]), Hkv or Hq
-  int32_t q_vec;                 // q rows 16-byte aligned 2-byte values: vector q loads
-  int32_t c_dtype;               // cache TMO_DTYPE_*
-  int32_t v_ch;                  // int4 caches: V pairs channels (else the rows of a page)
-  const void* mask;              // [B, S, mask_len] logit terms of the last keys, or null
-  int32_t mask_dtype;            // F32 / F16 / BF16
-  int32_t mask_len;
-  int64_t m_sb, m_ss;            // mask strides (sequence, token); last dim contiguous
-  int32_t splits;
-  int64_t split_tokens;          // multiple of 64
-  float* ws;                     // [B, Hkv, splits, ncols, Dv + 2] when splits > 1
-};
-
-// ------------------------------------------------------------------------------ small helpers
-
-
-__device__ __forceinline__ uint16_t bf16_bits_rne(float x) {
-  return __builtin_bit_cast(uint16_t, (__bf16)x);
-}
-__device__ __forceinline__ float bf16_value(uint16_t b) { return __uint_as_float((uint32_t)b << 16); }
-
-// Query element e as stored: a float, or an int8 / float8_e4m3fn code (its scale applies
-// separately: q_scale_of below).
-__device__ __forceinline__ float load_q(const AttnParams& p, int64_t e) {
-  switch (p.q_dtype) {
-    case TMO_DTYPE_BF16: return load1(BF16{}, p.q, e);
-    case TMO_DTYPE_F16: return load1(F16{}, p.q, e);
-    case TMO_DTYPE_I8: return (float)static_cast<const int8_t*>(p.q)[e];
-    case TMO_DTYPE_F8E4M3: return fp8_value(static_cast<const uint8_t*>(p.q)[e], 0);
-    default: return load1(F32{}, p.q, e);
-  }
-}
-
-// Scale of quantised q: the whole row's (per tensor, per token and head) -- `base` the row's
-// scale element i * qs_sb + row * qs_ss + hq * qs_sh -- or, per channel group, channel d's.
-__device__ __forceinline__ float q_row_scale(const AttnParams& p, int64_t base) {
-  if (p.qs_mode == 1) return scale_at(p.qs, 0, p.qs_bf16);
-  if (p.qs_mode == 2) return scale_at(p.qs, base, p.qs_bf16);
-  return 1.0f;
-}
-__device__ __forceinline__ float q_group_scale(const AttnParams& p, int64_t base, int d) {
-  return p.qs_mode == 3 ? scale_at(p.qs, base + d / p.qs_group, p.qs_bf16) : 1.0f;
-}
-
-// The block-table row of sequence i for query head hq (KV head hk): sparse-KV tables hold one
-// per KV head or per query head.
-__device__ __forceinline__ const int32_t* bt_row_of(const AttnParams& p, int64_t i, int hq, int hk) {
-  const int64_t r = p.bt_heads == 0 ? i : i * p.bt_heads + (p.bt_heads == p.Hq ? hq : hk);
-  return p.bt + r * p.max_blocks;
-}
-
-__device__ __forceinline__ void store_out(const AttnParams& p, int64_t e, float v) {
-  switch (p.o_dtype) {
-    case TMO_DTYPE_BF16: store1(BF16{}, p.out, e, v); break;
-    case TMO_DTYPE_F16: store1(F16{}, p.out, e, v); break;
-    default: store1(F32{}, p.out, e, v); break;
-  }
-}
-
-// Mask element e (a logit term, natural-log units) as fp32.
-__device__ __forceinline__ float mask_value(const AttnParams& p, int64_t e) {
-  switch (p.mask_dtype) {
-    case TMO_DTYPE_BF16: return load1(BF16{}, p.mask, e);
-    case TMO_DTYPE_F16: return load1(F16{}, p.mask, e);
-    default: return load1(F32{}, p.mask, e);
-  }
-}
-
-// Sequence i: its keys L (clamped to its block table), its query tokens nq (the first
-// min(nq, S) are computed) and the row of its token 0.
-struct Seq {
-  int64_t L, nq, row0;
-};
-
-__device__ __forceinline__ Seq seq_of(const AttnParams& p, int64_t i) {
-  Seq q;
-  int64_t L = p.lens[i];
-  const int64_t cap = p.max_blocks * (int64_t)p.BS;
-  if (L > cap) L = cap;
-  if (L < 0) L = 0;
-  q.L = L;
-  if (p.cu) {
-    q.row0 = p.cu[i];
-    q.nq = (int64_t)p.cu[i + 1] - q.row0;
-  } else {
-    q.row0 = 0;
-    q.nq = p.S;
-  }
-  return q;
-}
-
-// Token s of the sequence is computed: within S and nq, and (with cu_seq_q) a row of q.
-__device__ __forceinline__ bool token_valid(const AttnParams& p, const Seq& q, int64_t s) {
-  return s < p.S && s < q.nq && (!p.cu || (q.row0 + s >= 0 && q.row0 + s < p.total_q));
-}
-
-// Key range of the sequence (token 0's window start to L) and of split s within it.
-struct Range {
-  int64_t begin, end;
-};
-
-__device__ __forceinline__ Range token_range(const AttnParams& p, const Seq& q, int s) {
-  Range r;
-  const int64_t L = q.L;
-  int64_t j0 = 0;
-  if (p.window >= 0 && L - q.nq - p.window > 0) j0 = L - q.nq - p.window;
-  r.begin = j0 + (int64_t)s * p.split_tokens;
-  r.end = r.begin + p.split_tokens < L ? r.begin + p.split_tokens : L;
-  if (s == p.splits - 1) r.end = L;  // the last split takes any tokens past max_context_len
-  if (p.splits == 1) r.begin = j0;
-  return r;
-}
-
-// Final normalisation with the sink: m, l the column's maximum (base 2) and sum over its keys
-// (l = 0: none).  Returns the factor of the unnormalised accumulators and writes the lse.
-__device__ __forceinline__ float finish(const AttnParams& p, int hq, float m, float l, float* lse) {
-  float inv = l > 0.0f ? 1.0f / l : 0.0f;
-  float lg = l > 0.0f ? m + log2f(l) : -__builtin_inff();
-  if (p.sink) {
-    const float sk = p.sink[hq] * kLog2e;
-    if (l > 0.0f) {
-      const float mm = fmaxf(m, sk);
-      const float lt = l * __builtin_amdgcn_exp2f(m - mm) + __builtin_amdgcn_exp2f(sk - mm);
-      inv = __builtin_amdgcn_exp2f(m - mm) / lt;
-      lg = mm + log2f(lt);
-    } else {
-      lg = sk;
-    }
-  }
-  *lse = lg * kLn2;
-  return inv;
-}
-
-// Max / sum over the four lane groups (lanes l, l ^ 16, l ^ 32, l ^ 48) of a column.
-__device__ __forceinline__ float col_max(float v) {
-  v = fmaxf(v, __shfl_xor(v, 16, kWave));
-  return fmaxf(v, __shfl_xor(v, 32, kWave));
-}
-__device__ __forceinline__ float col_sum(float v) {
-  v += __shfl_xor(v, 16, kWave);
-  return v + __shfl_xor(v, 32, kWave);
-}
-
-// ------------------------------------------------------------------------------ MFMA kernel
-
-template <bool kF16>
-struct Mfma;
-template <>
-struct Mfma<false> {  // bf16 operands
-  typedef bf16x4 V4;
-  static __device__ __forceinline__ f32x4 run(V4 a, V4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
-  }
-  static __device__ __forceinline__ short bits(float x) { return (short)bf16_bits_rne(x); }
-  static __device__ __forceinline__ float value(short b) { return bf16_value((uint16_t)b); }
-};
-template <>
-struct Mfma<true> {  // f16 operands
-  typedef f16x4 V4;
-  static __device__ __forceinline__ f32x4 run(V4 a, V4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
-  }
-};
-
-// Four int8 codes (one dword) -> four f16 operands holding 1152 + code exactly: with
-// u = code + 128 (the byte with its top bit flipped), the f16 pattern 0x6400 | u is 1024 + u
-// (ulp 1 in [1024, 2048)), so two byte permutes build the four values.  The QK product then
-// carries 1152 * sum(q), which is subtracted per query column.
-constexpr float kCodeBias = 1152.0f;
-__device__ __forceinline__ f16x4 codes_f16(uint32_t w) {
-  const uint32_t u = w ^ 0x80808080u;
-  u32x2 h;
-  h[0] = __builtin_amdgcn_perm(0x64646464u, u, 0x04010400u);  // [u0, 0x64, u1, 0x64]
-  h[1] = __builtin_amdgcn_perm(0x64646464u, u, 0x04030402u);  // [u2, 0x64, u3, 0x64]
-  return __builtin_bit_cast(f16x4, h);
-}
-
-// Four float8_e4m3fn codes (one dword) -> four f16 operands holding their values exactly:
-// v_cvt_pk_f32_fp8 decodes two codes to fp32, v_cvt_pkrtz_f16_f32 packs two fp32 into f16
-// (every e4m3fn value -- at most 4 significant bits, 2^-9 .. 448 -- is an f16 value, so the
-// conversion's rounding never acts).
-__device__ __forceinline__ f16x4 fp8_f16(uint32_t w) {
-  typedef float f2 __attribute__((ext_vector_type(2)));
-  const f2 a = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, false);
-  const f2 b = __builtin_amdgcn_cvt_pk_f32_fp8((int)w, true);
-  u32x2 h;
-  h[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(a[0], a[1]));
-  h[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(b[0], b[1]));
-  return __builtin_bit_cast(f16x4, h);
-}
-
-// Eight int4 codes (one dword of a K row: byte b holds channels 2b (high nibble) and 2b + 1
-// (low nibble)) -> the f16 operands of channels 4h + {0, 2, 1, 3}, h = `half` (bytes 2h and
-// 2h + 1), as 2 + u / 8 with u = code + 8 (the nibble with its top bit flipped): the f16
-// pattern 0x4000 | u << 6 has exponent 1 and u in the top four mantissa bits, so the value
-// 3 + code / 8 is exact.  Each f16 pair is one byte permute (the two high or two low nibbles
-// into the pair's low bytes) and one shift-or.  The QK product then carries 3 * sum(q) and a
-// factor 1/8; the channel order within the operand is matched by q's.
-__device__ __forceinline__ f16x4 int4_f16(uint32_t w, int half) {
-  const uint32_t x = w ^ 0x88888888u;
-  const uint32_t hi = x & 0xf0f0f0f0u, lo = x & 0x0f0f0f0fu;
-  const uint32_t sel = half ? 0x0c030c02u : 0x0c010c00u;  // [byte 2h, 0, byte 2h + 1, 0]
-  u32x2 h;
-  h[0] = (__builtin_amdgcn_perm(hi, hi, sel) << 2) | 0x40004000u;  // channels 4h, 4h + 2
-  h[1] = (__builtin_amdgcn_perm(lo, lo, sel) << 6) | 0x40004000u;  // channels 4h + 1, 4h + 3
-  return __builtin_bit_cast(f16x4, h);
-}
-constexpr float kInt4Bias = 3.0f;
-// Channel of operand element e of QK MFMA m within the lane's run: int4 operands hold
-// channels 4m + {0, 2, 1, 3}
-__host__ __device__ constexpr int qk_channel(bool int4, int m, int e) {
-  return 4 * m + (int4 ? (((e & 1) << 1) | (e >> 1)) : e);
-}
 
 // kKind: 0 int8 caches (f16 QK, bf16 PV), 1 bf16 caches, 2 f16 caches, 3 float8_e4m3fn caches
 // (as int8: f16 QK against the exact code values, no bias; bf16 PV), 4 int4 pairs (K pairing
@@ -929,13 +668,16 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
   if (direct && grp == 0 && p.lse) p.lse[i * p.lse_sb + qrow * p.lse_ss + (int64_t)hq * p.lse_sh] = lse_v;
 }
 
-// Merge the splits of one (query token, query head): one wavefront per row.  Lane s holds
-// split s's (max, sum) and turns them into the split's weight sum_s * 2^(max_s - max), once;
-// the output channels then read each split's row once, weighted through a lane broadcast.
+// Merge the splits of one (query token, query head): one wavefront per row and 64 channels
+// (blockIdx.y).  Lane s holds split s's (max, sum) and turns them into the split's weight sum_s *
+// 2^(max_s - max), once; the output channels then read each split's row once, weighted through a
+// lane broadcast.
 __global__ __launch_bounds__(256) void attn_combine(AttnParams p) {
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t row = (int64_t)blockIdx.x * 4 + threadIdx.x / kWave;  // (i * S + s) * Hq + hq
   if (row >= (int64_t)p.B * p.S * p.Hq) return;
+  const int d = blockIdx.y * kWave + lane;
+  const int dc = d < p.Dv ? d : p.Dv - 1;
   const int64_t it = row / p.Hq;
   const int hq = (int)(row - it * p.Hq);
   const int64_t i = it / p.S;
@@ -962,11 +704,15 @@ __global__ __launch_bounds__(256) void attn_combine(AttnParams p) {
   const int last = live > 0 ? live - 1 : 0;
   const int64_t qrow = sq.row0 + tok;
   const int64_t orow = i * p.o_sb + qrow * p.o_ss + (int64_t)hq * p.o_sh;
-  constexpr int kBatch = 8;
+  constexpr int kBatch = 16;
   if (live <= kWave) {  // wave-uniform; every launch of the torch op (at most 63 splits)
     // lane s holds split s's (max, sum), loaded once; the values in batches of kBatch splits
+    // the first batch's values do not wait for the weights
     const int sc = lane < live ? lane : last;
     const float m_raw = base[sc * stride], l_raw = base[sc * stride + 1];
+    float v[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; ++k) v[k] = base[(k < live ? k : last) * stride + 2 + dc];
     const float m = lane < live ? m_raw : -__builtin_inff();
     float mx = m;
 #pragma unroll
@@ -977,23 +723,20 @@ __global__ __launch_bounds__(256) void attn_combine(AttnParams p) {
     for (int o = 32; o >= 1; o >>= 1) lt += __shfl_xor(lt, o, kWave);
     float lse_v;
     const float inv = finish(p, hq, mx, lt, &lse_v);
-    for (int d0 = 0; d0 < p.Dv; d0 += kWave) {
-      const int d = d0 + lane;
-      const int dc = d < p.Dv ? d : p.Dv - 1;
-      float o = 0.0f;
-      for (int k0 = 0; k0 < live; k0 += kBatch) {
-        float v[kBatch];
+    float o = 0.0f;
+    for (int k0 = 0; k0 < live; k0 += kBatch) {
+      if (k0 > 0) {
 #pragma unroll
         for (int k = 0; k < kBatch; ++k) v[k] = base[(k0 + k < live ? k0 + k : last) * stride + 2 + dc];
-#pragma unroll
-        for (int k = 0; k < kBatch; ++k) {
-          const float wk = __shfl(wgt, k0 + k < live ? k0 + k : 0, kWave);
-          if (k0 + k < live && wk != 0.0f) o += v[k] * wk;
-        }
       }
-      if (d < p.Dv) store_out(p, orow + d, o * inv);
+#pragma unroll
+      for (int k = 0; k < kBatch; ++k) {
+        const float wk = __shfl(wgt, k0 + k < live ? k0 + k : 0, kWave);
+        if (k0 + k < live && wk != 0.0f) o += v[k] * wk;
+      }
     }
-    if (lane == 0 && p.lse) p.lse[i * p.lse_sb + qrow * p.lse_ss + (int64_t)hq * p.lse_sh] = lse_v;
+    if (d < p.Dv) store_out(p, orow + d, o * inv);
+    if (d == 0 && p.lse) p.lse[i * p.lse_sb + qrow * p.lse_ss + (int64_t)hq * p.lse_sh] = lse_v;
     return;
   }
   float mx = -__builtin_inff();
@@ -1016,33 +759,29 @@ __global__ __launch_bounds__(256) void attn_combine(AttnParams p) {
   for (int o = 32; o >= 1; o >>= 1) lt += __shfl_xor(lt, o, kWave);
   float lse_v;
   const float inv = finish(p, hq, mx, lt, &lse_v);
-  for (int d0 = 0; d0 < p.Dv; d0 += kWave) {
-    const int d = d0 + lane;
-    const int dc = d < p.Dv ? d : p.Dv - 1;
-    float o = 0.0f;
-    for (int s0 = 0; s0 < live; s0 += kWave) {
-      const int sl = s0 + lane;
-      const int sc = sl < live ? sl : last;
-      const float m = sl < live ? base[sc * stride] : -__builtin_inff();
-      const float wgt = m != -__builtin_inff() ? base[sc * stride + 1] * __builtin_amdgcn_exp2f(m - mx) : 0.0f;
-      const int n = live - s0 < kWave ? live - s0 : kWave;
-      for (int k0 = 0; k0 < n; k0 += kBatch) {
-        float v[kBatch];
+  float o = 0.0f;
+  for (int s0 = 0; s0 < live; s0 += kWave) {
+    const int sl = s0 + lane;
+    const int sc = sl < live ? sl : last;
+    const float m = sl < live ? base[sc * stride] : -__builtin_inff();
+    const float wgt = m != -__builtin_inff() ? base[sc * stride + 1] * __builtin_amdgcn_exp2f(m - mx) : 0.0f;
+    const int n = live - s0 < kWave ? live - s0 : kWave;
+    for (int k0 = 0; k0 < n; k0 += kBatch) {
+      float v[kBatch];
 #pragma unroll
-        for (int k = 0; k < kBatch; ++k) {
-          const int s = s0 + (k0 + k < n ? k0 + k : n - 1);
-          v[k] = base[s * stride + 2 + dc];
-        }
+      for (int k = 0; k < kBatch; ++k) {
+        const int s = s0 + (k0 + k < n ? k0 + k : n - 1);
+        v[k] = base[s * stride + 2 + dc];
+      }
 #pragma unroll
-        for (int k = 0; k < kBatch; ++k) {
-          const float wk = __shfl(wgt, k0 + k < n ? k0 + k : 0, kWave);
-          if (k0 + k < n && wk != 0.0f) o += v[k] * wk;
-        }
+      for (int k = 0; k < kBatch; ++k) {
+        const float wk = __shfl(wgt, k0 + k < n ? k0 + k : 0, kWave);
+        if (k0 + k < n && wk != 0.0f) o += v[k] * wk;
       }
     }
-    if (d < p.Dv) store_out(p, orow + d, o * inv);
   }
-  if (lane == 0 && p.lse) p.lse[i * p.lse_sb + qrow * p.lse_ss + (int64_t)hq * p.lse_sh] = lse_v;
+  if (d < p.Dv) store_out(p, orow + d, o * inv);
+  if (d == 0 && p.lse) p.lse[i * p.lse_sb + qrow * p.lse_ss + (int64_t)hq * p.lse_sh] = lse_v;
 }
 
 // ------------------------------------------------------------------------------ generic kernel
@@ -1198,6 +937,12 @@ __global__ __launch_bounds__(256) void attn_generic(AttnParams p) {
 
 // ------------------------------------------------------------------------------ launch
 
+int launch_combine(const AttnParams& p, hipStream_t st) {
+  const int64_t rows = (int64_t)p.B * p.S * p.Hq;
+  const dim3 grid((unsigned)((rows + 3) / 4), (unsigned)((p.Dv + kWave - 1) / kWave));
+  return launch_kernel(attn_combine, grid, dim3(256), st, p);
+}
+
 template <int kD, int kKind, bool kSB>
 int launch_mfma_d(const AttnParams& p, bool qlo, hipStream_t st) {
   const dim3 grid((unsigned)(p.splits * p.ncb), (unsigned)p.Hkv, (unsigned)p.B), block(256);
@@ -1208,9 +953,7 @@ int launch_mfma_d(const AttnParams& p, bool qlo, hipStream_t st) {
   else
     rc = qlo ? launch_kernel(attn_mfma<kD, kKind, true, kSB, false>, grid, block, st, p)
              : launch_kernel(attn_mfma<kD, kKind, false, kSB, false>, grid, block, st, p);
-  if (rc != TMO_OK || p.splits == 1) return rc;
-  const int64_t rows = (int64_t)p.B * p.S * p.Hq;
-  return launch_kernel(attn_combine, dim3((unsigned)((rows + 3) / 4)), block, st, p);
+  return rc != TMO_OK || p.splits == 1 ? rc : launch_combine(p, st);
 }
 
 template <int kKind, bool kSB>
@@ -1443,7 +1186,12 @@ extern "C" int tmo_hip_cached_kv_attn(
   p.mask_len = (int32_t)mask_len;
   p.m_sb = mask_stride_batch;
   p.m_ss = mask_stride_token;
-  if (!mfma) {
+  // Latent caches: values and keys in one cache of 576 channels, 512 of them values
+  const bool latent = !quant && v_null && num_blocks > 0 && head_size == 576 &&
+                      head_size_v == 512 && k_cache_dim == 576 && block_size % 8 == 0 && p.q_vec &&
+                      al(k_cache, 16) &&
+                      (block_table_heads != num_q_heads || num_q_heads == num_kv_heads);
+  if (!mfma && !latent) {
     p.splits = 1;
     p.split_tokens = 1;
     const int64_t rows = batch * seq_q * num_q_heads;
@@ -1453,8 +1201,12 @@ extern "C" int tmo_hip_cached_kv_attn(
   // tokens per split: the context divided evenly, rounded up to whole 64-token steps (four
   // wavefronts x 16-token tiles)
   int64_t per = (max_context_len + splits - 1) / splits;
-  per = (per + 63) / 64 * 64;
+  per = latent ? (per + 31) / 32 * 32 : (per + 63) / 64 * 64;
   p.split_tokens = per > 0 ? per : 64;
+  if (latent) {
+    const int rc = launch_attn_latent(p, st);
+    return rc != TMO_OK || p.splits == 1 ? rc : launch_combine(p, st);
+  }
   // quantised caches: bf16 and f16 q, and int8 / float8_e4m3fn q codes, are exact f16 operands
   // after the power-of-two scaling; q folded with per-channel key scales or group-wise q
   // scales needs the lo operand

@@ -1369,10 +1369,20 @@ void single_query_cached_kv_attn(const torch::Tensor& q_ori, const torch::Tensor
   // with 8 spreads them.  configs[4]'s 512 (sequence, KV head) pairs, splits 1..10: 681, 726,
   // 595, 673, 556, 571, 550, 713, 561, 590 us (5 vs 7 repeated on one box: 560 vs 545).
   int64_t splits = 1;
-  const int64_t pairs = B * Hkv * ((seq_q * (Hq / Hkv) + 15) / 16);  // x column blocks
-  if (max_ctx > 0 && pairs < 3072) {
-    const int64_t want = (3072 + pairs - 1) / pairs;
-    const int64_t cap = (max_ctx + 255) / 256;
+  // Latent caches (one cache of 576 channels, 512 of them values): a workgroup holds a half or
+  // all of a CU's LDS and writes 16 or 32 rows of 514 floats, so fewer and longer splits: about
+  // 820 workgroups (one column block per workgroup, 512 fit the chip at once; 256 of the paired
+  // ones), at least 96 keys each.  32 sequences of 512..8192 keys with 16 heads, splits 9, 13,
+  // 17, 21, 25, 27, 47: 61, 52, 48, 45, 45, 57, 53 us; with 64 heads, 9, 13, 17, 21, 47: 115, 107,
+  // 109, 124, 144 us; one sequence of 8192, 16 heads, 9, 25, 47: 49, 26, 21 us.
+  const bool latent = !v_cache.has_value() && !int8 && !same_as_q && D == 576 && Dv == 512;
+  const int64_t cols = seq_q * (Hq / Hkv);
+  const int64_t groups = latent ? (cols <= 16 ? 1 : (cols + 31) / 32) : (cols + 15) / 16;
+  const int64_t pairs = B * Hkv * groups;  // workgroups of one split
+  const int64_t target = latent ? 820 : 3072, least = latent ? 96 : 256;
+  if (max_ctx > 0 && pairs < target) {
+    const int64_t want = latent ? std::max<int64_t>(1, target / pairs) : (target + pairs - 1) / pairs;
+    const int64_t cap = (max_ctx + least - 1) / least;
     splits = std::max<int64_t>(1, std::min<int64_t>({want, cap, 63}));
     if (splits > 1 && splits % 2 == 0) splits += splits + 1 <= cap ? 1 : -1;
   }

@@ -738,3 +738,37 @@ def test_attn_quantised_q_rejections(tmo, dev):
             call(q, odt, qs)
     with pytest.raises(RuntimeError):
         call(qb, torch.bfloat16, None, bt[:, None].expand(2, 3, -1).contiguous())
+
+
+# ---------------------------------------------------------------------------- latent caches
+
+@pytest.mark.parametrize("Hq,S,BS,dtype", [(16, 1, 16, torch.bfloat16), (16, 2, 64, torch.float16),
+                                           (3, 1, 8, torch.float16), (32, 1, 16, torch.float16),
+                                           (64, 1, 32, torch.bfloat16), (20, 3, 16, torch.bfloat16)])
+def test_attn_latent_edges(tmo, ref, dev, Hq, S, BS, dtype):
+    """The latent kernel (one 576-channel cache, 512 value channels, 16- and 32-column
+    workgroups): contexts at the edges of its 32- and 64-row tiles, a missing page, splits,
+    window, sink, ALiBi, mask; and rows past a context, whatever they hold, are not read."""
+    lens = [1, 31, 32, 33, 64, 65, 700]
+    case = W.attn_case(dtype, 150, kv="plain", B=7, Hq=Hq, Hkv=1, D=576, BS=BS,
+                       NB=7 * ((700 + BS - 1) // BS), max_ctx=700)
+    case.context_lens = torch.tensor(lens, dtype=torch.int32)
+    case.block_tables[6, 1] = -1
+    case.alibi = (0.5 ** torch.arange(1, Hq + 1, dtype=torch.float32)).repeat(7, 1)
+    one = W.AttnCase(case.q, case.k_cache, None, None, None, case.block_tables,
+                     case.context_lens, case.alibi)
+    q = W.attn_queries(dtype, 151, B=7, Hq=Hq, D=576, S=S)
+    sink = torch.linspace(-1.0, 2.0, Hq)
+    kw = dict(scale=576 ** -0.5, Dv=512)
+    clean, _ = run_attn_mq(tmo, ref, dev, one, q, sink=sink, **kw)
+    run_attn_mq(tmo, ref, dev, one, q, max_ctx=0, window=40, **kw)          # a single split
+    mask = torch.randn(7, S, 8 * S, generator=torch.Generator().manual_seed(152))
+    run_attn_mq(tmo, ref, dev, one, q, window=333, mask=mask, **kw)
+    for i, n in enumerate(lens):                                             # the last pages' rest
+        page = int(case.block_tables[i, (n - 1) // BS])
+        one.k_cache[page, 0, (n - 1) % BS + 1:] = float("nan")
+    out = tmo.single_query_cached_kv_attn(
+        q.to(dev), one.k_cache.to(dev), None, torch.empty(7, S, Hq, 512, dtype=dtype, device=dev),
+        one.block_tables.to(dev), one.context_lens.to(dev), None, None, one.alibi.to(dev), 700, -1,
+        -1, 576 ** -0.5, sink=sink.to(dev))
+    assert torch.equal(out.cpu().double(), clean)
