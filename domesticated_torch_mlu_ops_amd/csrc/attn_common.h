@@ -1,4 +1,5 @@
-// Shared by the attention kernels (decode_attn.hip, attn_latent.hip): the launch parameters, the
+// Shared by the attention kernels (decode_attn.hip, attn_latent.hip,
+// attn_chunk.hip): the launch parameters, the
 // sequence and key-range rules, the softmax's last step, and the MFMA operand conversions.
 #pragma once
 
@@ -54,6 +55,7 @@ struct AttnParams {
   int64_t qs_sb, qs_ss, qs_sh;   // q scale strides (sequence, token, head), as q's
   int32_t qs_group;              // mode 3: channels per scale (head_size / scale_num)
   int64_t bt_heads;              // block-table rows per sequence: 0 ([B, MB]), Hkv or Hq
+  int32_t o_vec;                 // 2-byte output rows 8-byte aligned: vector stores
   int32_t q_vec;                 // q rows 16-byte aligned 2-byte values: vector q loads
   int32_t c_dtype;               // cache TMO_DTYPE_*
   int32_t v_ch;                  // int4 caches: V pairs channels (else the rows of a page)
@@ -62,7 +64,8 @@ struct AttnParams {
   int32_t mask_len;
   int64_t m_sb, m_ss;            // mask strides (sequence, token); last dim contiguous
   int32_t splits;
-  int64_t split_tokens;          // multiple of 64
+  int32_t lone;                  // a sequence's only live split writes the output itself
+  int64_t split_tokens;          // multiple of 64 (latent caches: 32)
   float* ws;                     // [B, Hkv, splits, ncols, Dv + 2] when splits > 1
 };
 
@@ -144,6 +147,21 @@ __device__ __forceinline__ Seq seq_of(const AttnParams& p, int64_t i) {
   return q;
 }
 
+// The sequence of rank r by context length, longest first (batches of at most 64 sequences; r
+// itself in larger ones, which even out by their number).  Workgroups are dispatched in order, so
+// a long sequence that comes last would run on alone.
+__device__ __forceinline__ int64_t seq_by_length(const AttnParams& p, int r) {
+  if (p.B < 2 || p.B > kWave) return r;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int32_t own = lane < p.B ? p.lens[lane] : INT32_MIN;
+  int rank = 0;
+  for (int j = 0; j < p.B; ++j) {
+    const int32_t other = __builtin_amdgcn_readlane(own, j);
+    rank += other > own || (other == own && j < lane) ? 1 : 0;
+  }
+  return __builtin_ctzll(__ballot(lane < p.B && rank == r));
+}
+
 // Token s of the sequence is computed: within S and nq, and (with cu_seq_q) a row of q.
 __device__ __forceinline__ bool token_valid(const AttnParams& p, const Seq& q, int64_t s) {
   return s < p.S && s < q.nq && (!p.cu || (q.row0 + s >= 0 && q.row0 + s < p.total_q));
@@ -164,6 +182,14 @@ __device__ __forceinline__ Range token_range(const AttnParams& p, const Seq& q, 
   if (s == p.splits - 1) r.end = L;  // the last split takes any tokens past max_context_len
   if (p.splits == 1) r.begin = j0;
   return r;
+}
+
+// Splits of the sequence that hold keys: a prefix of the launch's (the others write nothing).
+__device__ __forceinline__ int live_splits(const AttnParams& p, const Seq& q) {
+  if (p.splits <= 1 || p.split_tokens <= 0) return p.splits;
+  const int64_t left = q.L - token_range(p, q, 0).begin;
+  const int64_t n = (left + p.split_tokens - 1) / p.split_tokens;
+  return left <= 0 ? 0 : (int)(n < p.splits ? n : p.splits);
 }
 
 // Final normalisation with the sink: m, l the column's maximum (base 2) and sum over its keys
@@ -267,8 +293,46 @@ __host__ __device__ constexpr int qk_channel(bool int4, int m, int e) {
   return 4 * m + (int4 ? (((e & 1) << 1) | (e >> 1)) : e);
 }
 
+// Two fp32 values as a packed 16-bit pair of the operand type, and the remainders as another.
+template <bool kF16>
+__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
+  if constexpr (kF16) {
+    const _Float16 ha = (_Float16)a, hb = (_Float16)b;
+    const _Float16 la = (_Float16)(a - (float)ha), lb = (_Float16)(b - (float)hb);
+    hi = (uint32_t)__builtin_bit_cast(uint16_t, ha) | ((uint32_t)__builtin_bit_cast(uint16_t, hb) << 16);
+    lo = (uint32_t)__builtin_bit_cast(uint16_t, la) | ((uint32_t)__builtin_bit_cast(uint16_t, lb) << 16);
+  } else {
+    typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    const f2 v = {a, b};
+    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf2));
+    const f2 r = {a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u)};
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf2));
+  }
+}
+
+// Output elements e .. e + 3 (one 8-byte store where the rows allow it).
+__device__ __forceinline__ void store_out4(const AttnParams& p, int64_t e, f32x4 v) {
+  if (p.o_vec) {
+    u32x2 w;
+    if (p.o_dtype == TMO_DTYPE_BF16) {
+      w[0] = pack2(BF16{}, v[0], v[1]);
+      w[1] = pack2(BF16{}, v[2], v[3]);
+    } else {
+      w[0] = pack2(F16{}, v[0], v[1]);
+      w[1] = pack2(F16{}, v[2], v[3]);
+    }
+    *reinterpret_cast<u32x2*>(static_cast<uint16_t*>(p.out) + e) = w;
+    return;
+  }
+#pragma unroll
+  for (int k = 0; k < 4; ++k) store_out(p, e + k, v[k]);
+}
+
 // The latent-cache kernel (attn_latent.hip): p.splits partials per column when > 1, as
 // attn_mfma leaves them.
 int launch_attn_latent(const AttnParams& p, hipStream_t st);
+// The many-column kernel (attn_chunk.hip), likewise; qlo: q needs a lo operand.
+int launch_attn_chunk(const AttnParams& p, bool qlo, hipStream_t st);
 
 }  // namespace tmo

@@ -69,24 +69,6 @@ __device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
                                                  __builtin_bit_cast(bf8, b), c, 0, 0, 0);
 }
 
-// Two fp32 values as a packed 16-bit pair of the operand type, and the remainders as another.
-template <bool kF16>
-__device__ __forceinline__ void split2(float a, float b, uint32_t& hi, uint32_t& lo) {
-  if constexpr (kF16) {
-    const _Float16 ha = (_Float16)a, hb = (_Float16)b;
-    const _Float16 la = (_Float16)(a - (float)ha), lb = (_Float16)(b - (float)hb);
-    hi = (uint32_t)__builtin_bit_cast(uint16_t, ha) | ((uint32_t)__builtin_bit_cast(uint16_t, hb) << 16);
-    lo = (uint32_t)__builtin_bit_cast(uint16_t, la) | ((uint32_t)__builtin_bit_cast(uint16_t, lb) << 16);
-  } else {
-    typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
-    typedef float f2 __attribute__((ext_vector_type(2)));
-    const f2 v = {a, b};
-    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf2));
-    const f2 r = {a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xffff0000u)};
-    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, bf2));
-  }
-}
-
 template <bool kF16, int kCB, bool kMask>
 __global__ __launch_bounds__(256 * kCB, 2) void attn_latent(AttnParams p) {
   constexpr int kT = 32 * kCB;        // tokens per LDS tile
@@ -377,9 +359,7 @@ __global__ __launch_bounds__(256 * kCB, 2) void attn_latent(AttnParams p) {
   }
   const int64_t orow = i * p.o_sb + qrow * p.o_ss + (int64_t)hq * p.o_sh;
 #pragma unroll
-  for (int b = 0; b < kLatVB; ++b)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) store_out(p, orow + d0 + 16 * b + e, acc[b][e] * inv);
+  for (int b = 0; b < kLatVB; ++b) store_out4(p, orow + d0 + 16 * b, acc[b] * inv);
   if (chq == 0 && grp == 0 && p.lse)
     p.lse[i * p.lse_sb + qrow * p.lse_ss + (int64_t)hq * p.lse_sh] = lse_v;
 }

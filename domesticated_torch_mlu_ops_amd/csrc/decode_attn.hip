@@ -688,15 +688,9 @@ __global__ __launch_bounds__(256) void attn_combine(AttnParams p) {
   const int c = tok * p.g + (hq - hk * p.g);
   const int64_t stride = (int64_t)p.ncols * (p.Dv + 2);
   const float* base = p.ws + ((i * p.Hkv + hk) * p.splits * (int64_t)p.ncols + c) * (p.Dv + 2);
-  // splits past the sequence's keys wrote nothing (the main kernel returned early): the
-  // non-empty splits are a prefix, of length `live`
-  const Range r0 = token_range(p, sq, 0);
-  int live = p.splits;
-  if (p.split_tokens > 0) {
-    const int64_t n = (sq.L - r0.begin + p.split_tokens - 1) / p.split_tokens;
-    live = (int)(n < p.splits ? n : p.splits);
-    if (live < 1 && p.splits > 0) live = r0.begin < sq.L ? 1 : 0;
-  }
+  // splits past the sequence's keys wrote nothing (the main kernel returned early)
+  const int live = live_splits(p, sq);
+  if (p.lone && live == 1) return;
   // Every load is unconditional (split and channel indices clamped into this column's rows of
   // the workspace; an empty split's row is read and given weight 0), so the loads of a batch
   // issue together.  Under the per-split weight test each row load waited for the previous
@@ -1154,6 +1148,8 @@ extern "C" int tmo_hip_cached_kv_attn(
             reinterpret_cast<uintptr_t>(q) % 16 == 0 &&
             p.q_sb % 8 == 0 && q_stride_token % 8 == 0 && q_stride_head % 8 == 0 &&
             (!quant || scale_mode != 2 || reinterpret_cast<uintptr_t>(k_scale) % 16 == 0);
+  p.o_vec = out_dtype != TMO_DTYPE_F32 && reinterpret_cast<uintptr_t>(out) % 8 == 0 &&
+            p.o_sb % 4 == 0 && out_stride_token % 4 == 0 && out_stride_head % 4 == 0;
   p.ws = static_cast<float*>(workspace);
   hipStream_t st = static_cast<hipStream_t>(stream);
 
@@ -1211,6 +1207,24 @@ extern "C" int tmo_hip_cached_kv_attn(
   // after the power-of-two scaling; q folded with per-channel key scales or group-wise q
   // scales needs the lo operand
   const bool qlo = scale_mode == 2 || p.qs_mode == 3;
+  // Four column blocks and more (49 columns) take attn_chunk, which unpacks a key once for 64 or
+  // 128 columns.  8 KV heads x 128, int8 pages, contexts of 512..8192, attn_mfma against it: 32
+  // columns of 4 / 32 sequences 53 / 160 against 54 / 183 us, 64 columns 72 / 267 against 55 /
+  // 193, 128 columns (32 sequences) 492 against 212, 2048 columns of 8 sequences 1210 against 437.
+  // It indexes cache rows and scales with 32 bits and has no mask or ALiBi terms.
+  auto scale_span = [&](int64_t sb, int64_t sh) {
+    return num_blocks * sb + num_kv_heads * sh + block_size;
+  };
+  if (mfma && ncb >= 4 && !mask && !alibi_slopes &&
+      num_kv_heads * splits * ((p.ncols + 63) / 64) <= 0x7fffffffLL &&
+      num_blocks * num_kv_heads * block_size <= 0x7fffffffLL &&
+      (!quant || scale_mode != 1 ||
+       (scale_span(k_scale_stride_block, k_scale_stride_head) <= 0x7fffffffLL &&
+        scale_span(v_scale_stride_block, v_scale_stride_head) <= 0x7fffffffLL))) {
+    p.lone = 1;
+    const int rc = launch_attn_chunk(p, qlo, st);
+    return rc != TMO_OK || p.splits == 1 ? rc : launch_combine(p, st);
+  }
   if (cache_dtype == TMO_DTYPE_I8)
     return p.s_bf16 ? launch_mfma<0, true>(p, qlo, st) : launch_mfma<0, false>(p, qlo, st);
   if (cache_dtype == TMO_DTYPE_F8E4M3)

@@ -772,3 +772,47 @@ def test_attn_latent_edges(tmo, ref, dev, Hq, S, BS, dtype):
         one.block_tables.to(dev), one.context_lens.to(dev), None, None, one.alibi.to(dev), 700, -1,
         -1, 576 ** -0.5, sink=sink.to(dev))
     assert torch.equal(out.cpu().double(), clean)
+
+
+# ---------------------------------------------------------------------------- many query columns
+
+@pytest.mark.parametrize("kv,D,Hq,S,dtype,scales", [
+    ("int8_token", 128, 8, 13, torch.bfloat16, torch.float32),     # 52 columns: one wavefront short
+    ("int8_token", 128, 8, 33, torch.float16, torch.bfloat16),     # 132: a second workgroup
+    ("int8_channel", 128, 8, 17, torch.bfloat16, torch.float32),   # q folded: lo operand
+    ("int8_token", 64, 16, 40, torch.bfloat16, torch.float32),
+    ("fp8_token", 256, 8, 16, torch.bfloat16, torch.float32),
+    ("fp8_channel", 64, 8, 16, torch.float16, torch.bfloat16),
+    ("int4_token", 128, 8, 20, torch.bfloat16, torch.float32),
+    ("int4_channel", 256, 8, 13, torch.float16, torch.float32),
+    ("plain", 128, 8, 32, torch.bfloat16, None),
+    ("plain", 256, 2, 64, torch.float16, None)])
+def test_attn_many_columns(tmo, ref, dev, kv, D, Hq, S, dtype, scales):
+    """The many-column kernel over its kinds and head sizes: contexts at the edges of its 32- and
+    64-key tiles, missing pages, a window, a sink, a negative softmax scale, ragged counts with
+    rows of no sequence, one split and several."""
+    lens = [70, 1, 16, 64, 65, 127, 1500]
+    case = W.attn_case(dtype, 160 + D, kv=kv, B=7, Hq=Hq, Hkv=2, D=D, BS=16, NB=700, max_ctx=1500,
+                       scale_dtype=scales or torch.float32)
+    case.context_lens = torch.tensor(lens, dtype=torch.int32)
+    case.block_tables[6, 40:42] = -1
+    q = W.attn_queries(dtype, 161, B=7, Hq=Hq, D=D, S=S)
+    scale = D ** -0.5
+    run_attn_mq(tmo, ref, dev, case, q, scale=scale, sink=torch.linspace(-1.0, 2.0, Hq))
+    run_attn_mq(tmo, ref, dev, case, q, scale=-0.5 * scale, window=50, max_ctx=0)
+    counts = [S, 1, min(16, S), 0, S - 3, 3, S]
+    q3, cu = W.attn_queries(dtype, 162, B=7, Hq=Hq, D=D, counts=counts)
+    run_attn_mq(tmo, ref, dev, case, torch.cat([q3, q3[:2]]), cu=cu, scale=scale, max_seq_q=S)
+
+
+def test_attn_many_columns_quantised_q_and_sparse_tables(tmo, ref, dev):
+    """Quantised q (per token, and per channel group: lo operand) and per-KV-head block tables on
+    the many-column kernel."""
+    case = W.attn_case(torch.bfloat16, 170, kv="int8_token", B=3, Hq=8, Hkv=2, D=128, NB=96,
+                       max_ctx=200)
+    g = torch.Generator().manual_seed(171)
+    case.block_tables = torch.stack([torch.randperm(96, generator=g)[:26].reshape(2, 13)
+                                     for _ in range(3)]).to(torch.int32)
+    q = _q_codes(torch.int8, (3, 20, 8, 128), 172)
+    for form in ("token", "group"):
+        run_attn_mq(tmo, ref, dev, case, q, q_scale=_q_scale(form, (3, 20, 8), 173))
