@@ -1162,8 +1162,9 @@ extern "C" int tmo_hip_cached_kv_attn(
   // see attn_mfma), so an empty cache takes attn_generic, whose loads are all under the page
   // check: every output row is then 0 and its lse -inf (nothing to attend to).
   // int4 pages: K rows of head_size / 2 bytes, V pairing rows (pair rows of head_size bytes)
-  bool mfma = num_blocks > 0 && (head_size == 64 || head_size == 128 || head_size == 256) &&
-              head_size_v == head_size &&
+  const bool whole = head_size == 64 || head_size == 128 || head_size == 256;
+  const bool part = (head_size == 80 && !int4) || head_size == 96;  // attn_chunk only
+  bool mfma = num_blocks > 0 && (whole || part) && head_size_v == head_size &&
               k_cache_dim == (int4 ? head_size / 2 : head_size) && v_cache_dim == head_size &&
               !(int4 && v_pair_channels) && block_size % 16 == 0 && al(k_cache, 16) &&
               al(v_cache, 16) && q_dtype != TMO_DTYPE_F32 &&
@@ -1187,7 +1188,24 @@ extern "C" int tmo_hip_cached_kv_attn(
                       head_size_v == 512 && k_cache_dim == 576 && block_size % 8 == 0 && p.q_vec &&
                       al(k_cache, 16) &&
                       (block_table_heads != num_q_heads || num_q_heads == num_kv_heads);
-  if (!mfma && !latent) {
+  // Four column blocks and more (49 columns) take attn_chunk, which unpacks a key once for 64 or
+  // 128 columns.  8 KV heads x 128, int8 pages, contexts of 512..8192, attn_mfma against it: 32
+  // columns of 4 / 32 sequences 53 / 160 against 54 / 183 us, 64 columns 72 / 267 against 55 /
+  // 193, 128 columns (32 sequences) 492 against 212, 2048 columns of 8 sequences 1210 against 437.
+  // Head sizes 80 and 96 take it with any number of columns (attn_mfma has no instance of them),
+  // but for fp32 outputs, where the VALU kernel's fp32 probabilities show: 16 sequences of
+  // 512..8192 int8 keys, 32 heads x 96, one token each, 12486 us there, 104 here.
+  // It indexes cache rows and scales with 32 bits and has no mask or ALiBi terms.
+  auto scale_span = [&](int64_t sb, int64_t sh) {
+    return num_blocks * sb + num_kv_heads * sh + block_size;
+  };
+  const bool chunk = mfma && (whole ? ncb >= 4 : out_dtype != TMO_DTYPE_F32) && !mask && !alibi_slopes &&
+                     num_kv_heads * splits * ((p.ncols + 63) / 64) <= 0x7fffffffLL &&
+                     num_blocks * num_kv_heads * block_size <= 0x7fffffffLL &&
+                     (!quant || scale_mode != 1 ||
+                      (scale_span(k_scale_stride_block, k_scale_stride_head) <= 0x7fffffffLL &&
+                       scale_span(v_scale_stride_block, v_scale_stride_head) <= 0x7fffffffLL));
+  if (!(mfma && whole) && !chunk && !latent) {
     p.splits = 1;
     p.split_tokens = 1;
     const int64_t rows = batch * seq_q * num_q_heads;
@@ -1207,20 +1225,7 @@ extern "C" int tmo_hip_cached_kv_attn(
   // after the power-of-two scaling; q folded with per-channel key scales or group-wise q
   // scales needs the lo operand
   const bool qlo = scale_mode == 2 || p.qs_mode == 3;
-  // Four column blocks and more (49 columns) take attn_chunk, which unpacks a key once for 64 or
-  // 128 columns.  8 KV heads x 128, int8 pages, contexts of 512..8192, attn_mfma against it: 32
-  // columns of 4 / 32 sequences 53 / 160 against 54 / 183 us, 64 columns 72 / 267 against 55 /
-  // 193, 128 columns (32 sequences) 492 against 212, 2048 columns of 8 sequences 1210 against 437.
-  // It indexes cache rows and scales with 32 bits and has no mask or ALiBi terms.
-  auto scale_span = [&](int64_t sb, int64_t sh) {
-    return num_blocks * sb + num_kv_heads * sh + block_size;
-  };
-  if (mfma && ncb >= 4 && !mask && !alibi_slopes &&
-      num_kv_heads * splits * ((p.ncols + 63) / 64) <= 0x7fffffffLL &&
-      num_blocks * num_kv_heads * block_size <= 0x7fffffffLL &&
-      (!quant || scale_mode != 1 ||
-       (scale_span(k_scale_stride_block, k_scale_stride_head) <= 0x7fffffffLL &&
-        scale_span(v_scale_stride_block, v_scale_stride_head) <= 0x7fffffffLL))) {
+  if (chunk) {
     p.lone = 1;
     const int rc = launch_attn_chunk(p, qlo, st);
     return rc != TMO_OK || p.splits == 1 ? rc : launch_combine(p, st);

@@ -785,6 +785,13 @@ def test_attn_latent_edges(tmo, ref, dev, Hq, S, BS, dtype):
     ("fp8_channel", 64, 8, 16, torch.float16, torch.bfloat16),
     ("int4_token", 128, 8, 20, torch.bfloat16, torch.float32),
     ("int4_channel", 256, 8, 13, torch.float16, torch.float32),
+    ("int8_token", 80, 8, 2, torch.float16, torch.float32),        # 8 columns, padded channels
+    ("int8_channel", 80, 8, 9, torch.bfloat16, torch.float32),
+    ("fp8_token", 80, 2, 1, torch.bfloat16, torch.bfloat16),
+    ("int4_token", 96, 8, 20, torch.bfloat16, torch.float32),
+    ("int8_token", 96, 8, 1, torch.bfloat16, torch.float32),
+    ("plain", 80, 8, 33, torch.float16, None),
+    ("plain", 96, 8, 1, torch.bfloat16, None),
     ("plain", 128, 8, 32, torch.bfloat16, None),
     ("plain", 256, 2, 64, torch.float16, None)])
 def test_attn_many_columns(tmo, ref, dev, kv, D, Hq, S, dtype, scales):
@@ -800,7 +807,7 @@ def test_attn_many_columns(tmo, ref, dev, kv, D, Hq, S, dtype, scales):
     scale = D ** -0.5
     run_attn_mq(tmo, ref, dev, case, q, scale=scale, sink=torch.linspace(-1.0, 2.0, Hq))
     run_attn_mq(tmo, ref, dev, case, q, scale=-0.5 * scale, window=50, max_ctx=0)
-    counts = [S, 1, min(16, S), 0, S - 3, 3, S]
+    counts = [S, 1, min(16, S), 0, max(0, S - 3), min(3, S), S]
     q3, cu = W.attn_queries(dtype, 162, B=7, Hq=Hq, D=D, counts=counts)
     run_attn_mq(tmo, ref, dev, case, torch.cat([q3, q3[:2]]), cu=cu, scale=scale, max_seq_q=S)
 
