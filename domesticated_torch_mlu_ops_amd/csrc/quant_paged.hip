@@ -56,6 +56,8 @@ __device__ __forceinline__ bool locate_slot(const QuantPagedParams& p, int32_t s
   return true;
 }
 
+constexpr int kPartRow = 128;  // flag beside a lane count (a power of two <= 64)
+
 #ifndef TMO_QUANT_TOKENS_PER_THREAD
 #define TMO_QUANT_TOKENS_PER_THREAD 1
 #endif
@@ -74,12 +76,20 @@ constexpr int kTokensPerThread = TMO_QUANT_TOKENS_PER_THREAD;
 // owns kTokensPerThread * blockDim.x / G consecutive tokens of one head.
 // Every load of the lane group (slots, K rows, V rows) is issued before the first wait: the
 // input address does not depend on the slot, only the store address does.
-template <class Tag, int G, int V, bool kFp8>
+//
+// GP is G, plus kPartRow where the row has fewer than G vectors (head sizes 80, 96, ...): the
+// lanes past the row read its last vector again, which leaves the maximum alone, and store
+// nothing.  9973 tokens x 8 heads x 96 fp16 -> fp8: 44.5 us on the scalar kernel, 13.1 here.
+template <class Tag, int GP, int V, bool kFp8>
 __global__ __launch_bounds__(256) void quant_paged_vec(QuantPagedParams p) {
+  constexpr int G = GP & (kPartRow - 1);
+  constexpr bool kPart = GP >= kPartRow;
+  static_assert(!kPart || V == 1, "part rows hold one vector per lane");
   const int kGroups = blockDim.x / G;  // lane groups per workgroup
   constexpr int kPer = Tag::kPerVec;
   constexpr int kT = kTokensPerThread;
-  const int lane = threadIdx.x & (G - 1);
+  const int own = threadIdx.x & (G - 1);
+  const int lane = kPart ? min(own, p.head_dim / kPer - 1) : own;
 #if TMO_QUANT_XCD
   // XCD-aware order: the tile's per-token scale lines (64 bytes of each of two heads in one
   // 128-byte line for block size 16) are written whole from one L2
@@ -134,6 +144,7 @@ __global__ __launch_bounds__(256) void quant_paged_vec(QuantPagedParams p) {
         int8_t* row = p.cache[kv] + page_row * p.head_dim;
 #pragma unroll
         for (int i = 0; i < V; ++i) {
+          if (kPart && own != lane) continue;
           int8_t* dst = row + (lane + i * G) * kPer;
           uint32_t c[kPer / 4];
           if constexpr (kFp8) {
@@ -152,7 +163,7 @@ __global__ __launch_bounds__(256) void quant_paged_vec(QuantPagedParams p) {
         }
         // A plain store: the 4-byte scales of neighbouring heads share a line, which the L2 of
         // the tile's XCD merges (configs[0]: 2.96 -> 2.69 us per call, larger calls unchanged)
-        if (lane == 0) p.scale[kv][page_row] = rs.s;
+        if (own == 0) p.scale[kv][page_row] = rs.s;
       }
     }
   }
@@ -215,14 +226,17 @@ struct StaticParams {
 // lane always covers the same kPerVec channels of its head, so it loads their scales once
 // and computes the reciprocals once for its kT tokens.  There is no row reduction and no
 // scale store.
-template <class Tag, int G, bool kFp8>
+template <class Tag, int GP, bool kFp8>
 __global__ __launch_bounds__(256) void quant_paged_static_vec(StaticParams sp) {
+  constexpr int G = GP & (kPartRow - 1);  // part rows as in quant_paged_vec
+  constexpr bool kPart = GP >= kPartRow;
   const QuantPagedParams& p = sp.q;
   const StaticScales& sc = sp.sc;
   constexpr int kGroups = 256 / G;
   constexpr int kPer = Tag::kPerVec;
   constexpr int kT = TMO_STATIC_TOKENS_PER_THREAD;
-  const int lane = threadIdx.x & (G - 1);
+  const int own = threadIdx.x & (G - 1);
+  const int lane = kPart ? min(own, p.head_dim / kPer - 1) : own;
 #if TMO_QUANT_XCD
   int h;
   int64_t tile;
@@ -306,6 +320,7 @@ __global__ __launch_bounds__(256) void quant_paged_static_vec(StaticParams sp) {
         float v[kPer], q[kPer];
         unpack(Tag{}, w[j][kv], v);
         static_quotients<kPer, kFp8>(v, s[kv], y[kv], fast[kv], q);
+        if (kPart && own != lane) continue;
         uint32_t c[kPer / 4];
         encode_static<kPer, kFp8>(q, c);
         int8_t* dst = p.cache[kv] + page_row * p.head_dim + lane * kPer;
@@ -351,13 +366,20 @@ __global__ __launch_bounds__(256) void quant_paged_static_generic(StaticParams s
   }
 }
 
+// Lanes of a row of nvec vectors: the next power of two.
+int lanes_for(int nvec) {
+  int g = 1;
+  while (g < nvec) g *= 2;
+  return g;
+}
+
 template <class Tag, bool kFp8>
 int launch_static(const StaticParams& sp, hipStream_t stream) {
   const QuantPagedParams& p = sp.q;
   const StaticScales& sc = sp.sc;
   constexpr int kPer = Tag::kPerVec;
   const int nvec = p.head_dim % kPer == 0 ? p.head_dim / kPer : 0;
-  bool vec = nvec >= 1 && nvec <= kWave && (nvec & (nvec - 1)) == 0;
+  bool vec = nvec >= 1 && nvec <= kWave;
   for (int kv = 0; kv < p.nkv && vec; ++kv) {
     vec = (reinterpret_cast<uintptr_t>(p.src[kv]) % 16 == 0) &&
           ((p.stride_tok[kv] * Tag::kBytes) % 16 == 0) &&
@@ -365,7 +387,8 @@ int launch_static(const StaticParams& sp, hipStream_t stream) {
           (reinterpret_cast<uintptr_t>(p.cache[kv]) % 8 == 0) &&
           (reinterpret_cast<uintptr_t>(sc.chan[kv]) % 16 == 0);  // null passes
   }
-  const int G = vec ? nvec : kWave;
+  const int G = vec ? lanes_for(nvec) : kWave;  // a power of two; more than nvec: a part row
+  const bool part = vec && G != nvec;
   const int rows = vec ? (256 / G) * TMO_STATIC_TOKENS_PER_THREAD : 256 / kWave;
   const int64_t tiles = (p.num_tokens + rows - 1) / rows;
   const int64_t blocks = tiles * p.heads;
@@ -376,7 +399,12 @@ int launch_static(const StaticParams& sp, hipStream_t stream) {
     return launch_kernel(quant_paged_static_generic<Tag, kFp8>, dim3((unsigned)blocks), block,
                          stream, sp);
   const dim3 grid((unsigned)vec_blocks);
-  switch (G) {
+  switch (G | (part ? kPartRow : 0)) {
+    case 4 | kPartRow: return launch_kernel(quant_paged_static_vec<Tag, 4 | kPartRow, kFp8>, grid, block, stream, sp);
+    case 8 | kPartRow: return launch_kernel(quant_paged_static_vec<Tag, 8 | kPartRow, kFp8>, grid, block, stream, sp);
+    case 16 | kPartRow: return launch_kernel(quant_paged_static_vec<Tag, 16 | kPartRow, kFp8>, grid, block, stream, sp);
+    case 32 | kPartRow: return launch_kernel(quant_paged_static_vec<Tag, 32 | kPartRow, kFp8>, grid, block, stream, sp);
+    case 64 | kPartRow: return launch_kernel(quant_paged_static_vec<Tag, 64 | kPartRow, kFp8>, grid, block, stream, sp);
     case 1: return launch_kernel(quant_paged_static_vec<Tag, 1, kFp8>, grid, block, stream, sp);
     case 2: return launch_kernel(quant_paged_static_vec<Tag, 2, kFp8>, grid, block, stream, sp);
     case 4: return launch_kernel(quant_paged_static_vec<Tag, 4, kFp8>, grid, block, stream, sp);
@@ -389,6 +417,16 @@ int launch_static(const StaticParams& sp, hipStream_t stream) {
 
 template <class Tag, int V, bool kFp8>
 int launch_vec(const QuantPagedParams& p, int G, dim3 grid, dim3 block, hipStream_t stream) {
+  if constexpr (V == 1) {
+    switch (G) {
+      case 4 | kPartRow: return launch_kernel(quant_paged_vec<Tag, 4 | kPartRow, 1, kFp8>, grid, block, stream, p);
+      case 8 | kPartRow: return launch_kernel(quant_paged_vec<Tag, 8 | kPartRow, 1, kFp8>, grid, block, stream, p);
+      case 16 | kPartRow: return launch_kernel(quant_paged_vec<Tag, 16 | kPartRow, 1, kFp8>, grid, block, stream, p);
+      case 32 | kPartRow: return launch_kernel(quant_paged_vec<Tag, 32 | kPartRow, 1, kFp8>, grid, block, stream, p);
+      case 64 | kPartRow: return launch_kernel(quant_paged_vec<Tag, 64 | kPartRow, 1, kFp8>, grid, block, stream, p);
+      default: break;
+    }
+  }
   switch (G) {
     case 1: return launch_kernel(quant_paged_vec<Tag, 1, V, kFp8>, grid, block, stream, p);
     case 2: return launch_kernel(quant_paged_vec<Tag, 2, V, kFp8>, grid, block, stream, p);
@@ -405,7 +443,8 @@ int launch(const QuantPagedParams& p, hipStream_t stream) {
   constexpr int kPer = Tag::kPerVec;
   bool vec = (p.head_dim % kPer) == 0;
   const int nvec = vec ? p.head_dim / kPer : 0;  // 16-byte vectors per row
-  vec = vec && nvec >= 1 && nvec <= 64 * TMO_QUANT_VEC_PER_LANE && (nvec & (nvec - 1)) == 0;
+  const bool pow2 = nvec > 0 && (nvec & (nvec - 1)) == 0;
+  vec = vec && nvec >= 1 && nvec <= (pow2 ? 64 * TMO_QUANT_VEC_PER_LANE : 64);
   for (int kv = 0; kv < p.nkv && vec; ++kv) {
     vec = (reinterpret_cast<uintptr_t>(p.src[kv]) % 16 == 0) &&
           ((p.stride_tok[kv] * Tag::kBytes) % 16 == 0) &&
@@ -413,8 +452,8 @@ int launch(const QuantPagedParams& p, hipStream_t stream) {
           (reinterpret_cast<uintptr_t>(p.cache[kv]) % 8 == 0);
   }
   // V vectors per lane when the row has at least 4 * V of them, else one
-  const int V = (vec && nvec >= 4 * TMO_QUANT_VEC_PER_LANE) ? TMO_QUANT_VEC_PER_LANE : 1;
-  const int G = vec ? nvec / V : kWave;
+  const int V = (vec && pow2 && nvec >= 4 * TMO_QUANT_VEC_PER_LANE) ? TMO_QUANT_VEC_PER_LANE : 1;
+  const int G = vec ? lanes_for(nvec / V) : kWave;  // a power of two; more than nvec: a part row
   // Decode-sized launches (fewer than two 256-thread workgroups per CU of a 256-CU part) use
   // 64-thread workgroups: four times as many workgroups spread the row loads and the
   // scattered page stores over more CUs.  configs[1] (256 tokens x 8 heads, 128 -> 512
@@ -436,7 +475,7 @@ int launch(const QuantPagedParams& p, hipStream_t stream) {
   const dim3 block(256);
   if (!vec) return launch_kernel(quant_paged_generic<Tag, kFp8>, dim3((unsigned)blocks), block, stream, p);
   const dim3 grid((unsigned)vec_blocks), vblock(wg);
-  if (V == 1) return launch_vec<Tag, 1, kFp8>(p, G, grid, vblock, stream);
+  if (V == 1) return launch_vec<Tag, 1, kFp8>(p, pow2 ? G : G | kPartRow, grid, vblock, stream);
   return launch_vec<Tag, TMO_QUANT_VEC_PER_LANE, kFp8>(p, G, grid, vblock, stream);
 }
 

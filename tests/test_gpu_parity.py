@@ -136,6 +136,24 @@ def test_quant_shapes_and_block_sizes(tmo, ref, dev, dtype, D, BS):
     check_quant(tmo, ref, dev, case)
 
 
+PART_DIMS = [12, 24, 40, 72, 80, 96, 120, 144, 192, 248, 264, 504]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("D", PART_DIMS)
+def test_quant_part_rows(tmo, ref, dev, dtype, D):
+    """Head sizes that leave lanes of a row's group idle: the row maximum placed in every lane,
+    dynamic and per-channel static scales, int8 and fp8 pages."""
+    case = _case(f"part D={D}", 70, 3, D, 40, 16, dtype, seed=D, neg_frac=0.1)
+    k = case.k.clone()
+    for t in range(70):
+        k[t, :, (t * 7) % D] = 50.0 * (1 if t % 2 else -1)
+    ks, vs = (0.01 + 0.2 * torch.rand(3, D, generator=torch.Generator().manual_seed(s)) for s in (1, 2))
+    for cdt in (torch.int8, torch.float8_e4m3fn):
+        check_quant(tmo, ref, dev, case, k=k, cache_dtype=cdt)
+        check_offline(tmo, ref, dev, f"part D={D}", k, case.v, ks, vs, case.slot_mapping, 40, 16, cdt)
+
+
 def test_quant_k_only_and_strided_views(tmo, ref, dev):
     """v=None, and k/v as column views of a fused [T, 3H, D] qkv tensor."""
     T, H, D = 64, 4, 128
