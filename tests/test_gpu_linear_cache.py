@@ -328,6 +328,24 @@ def test_dequant_from_linear_cache_widths(tmo, ref, dev, D):
     _dequant_both(tmo, ref, dev, case, torch.float16, 0, with_v=False)
 
 
+@pytest.mark.parametrize("packed,offsets", [(True, False), (True, True), (False, True)])
+@pytest.mark.parametrize("D", [24, 40, 80, 120, 144, 248, 264, 504])
+def test_linear_part_rows(tmo, ref, dev, D, packed, offsets):
+    """Head sizes that leave lanes of a row's group idle: the quantisers (dynamic and static,
+    token-major and sequence-major grids) and the dequant."""
+    case = W.linear_case(torch.float16, 64 + D, packed=packed, offsets=offsets, D=D)
+    for t in range(case.key.shape[0]):
+        case.key[t, ..., (7 * t) % D] = 30.0 if t % 2 else -30.0   # the row maximum in every lane
+    for cdt in (torch.int8, torch.float8_e4m3fn):
+        _quant_both(tmo, ref, dev, case, cdt)
+        _offline_both(tmo, ref, dev, case, cdt, 0)
+    _offline_both(tmo, ref, dev, case, torch.int8, 1, with_v=False)
+    if packed:
+        for mode in (0, 1):
+            _dequant_both(tmo, ref, dev, case, torch.bfloat16, mode)
+            _dequant_both(tmo, ref, dev, case, torch.float32, mode, with_v=False)
+
+
 def _paged_view(case, NB_per=4):
     """Re-cut the case's cache geometry into pages: block_rows = cache_len // NB_per."""
     case.cache_len //= NB_per
