@@ -439,10 +439,17 @@ __global__ __launch_bounds__(256) void dequant_page_list(DequantParams p, PageEn
   list[page_start + j] = e;
 }
 
-template <class Tag, int kMode, int kKV, int kCS>
+//
+// Rows whose 8-code chunks are no power of two (head sizes 80, 96, ...; part rows, kMode with
+// kPartRow) count as the next power of two of units: the units past a row read its last chunk
+// and write nothing.
+constexpr int kPartRow = 2;  // flag beside the scale mode
+template <class Tag, int kModeP, int kKV, int kCS>
 __global__ __launch_bounds__(256) void dequant_paged_list(DequantParams p,
                                                           const PageEntry* __restrict__ list,
                                                           const int64_t* __restrict__ total) {
+  constexpr int kMode = kModeP & (kPartRow - 1);
+  constexpr bool kPart = kModeP >= kPartRow;
   // XCD-aware item order: workgroups are dispatched round-robin over the 8 XCDs, so workgroup
   // b runs on XCD b % 8.  All items of one page go to the same XCD (page = 8 * (slot / parts)
   // + b % 8, part = slot % parts, slot = b / 8), where they share its L2 -- one fetch of the
@@ -453,10 +460,12 @@ __global__ __launch_bounds__(256) void dequant_paged_list(DequantParams p,
   const uint32_t slot = blockIdx.x / kXcds;
   int64_t w = (int64_t)(slot >> part_shift) * kXcds + blockIdx.x % kXcds;
   const int u = ((int)(slot & ((1u << part_shift) - 1)) << 8) + threadIdx.x;
-  const int u8 = p.u_shift + 1;  // log2(head_dim / 8)
+  const int u8 = p.u_shift + 1;  // log2 of the units of a row (head_dim / 8 of them whole)
   const int o = (u >> u8) & (p.block_size - 1);
   const int h = u >> (u8 + p.bs_shift);
-  const int d0 = (u & ((1 << u8) - 1)) * 8;
+  const int own = (u & ((1 << u8) - 1)) * 8;
+  const int d0 = kPart ? min(own, p.head_dim - 8) : own;
+  const int64_t code0 = kPart ? (int64_t)(u >> u8) * p.head_dim + d0 : (int64_t)u * 8;
   const int64_t page_codes = (int64_t)p.heads * p.block_size * p.head_dim;
   const int64_t page_rows = (int64_t)p.heads * p.block_size;
   // the entry is read before the count (the list holds at least `stride` entries), so the
@@ -468,7 +477,7 @@ __global__ __launch_bounds__(256) void dequant_paged_list(DequantParams p,
     if (w != first) e = list[w];
     if (e.blk < 0) continue;  // workgroup-uniform
     const int64_t row = e.row0 + o;
-    const bool ok = o < e.ntok && row >= 0 && row < p.total_rows;
+    const bool ok = o < e.ntok && row >= 0 && row < p.total_rows && (!kPart || own == d0);
     // every unit of a valid page lies inside the caches, so the loads are unconditional (a
     // tail token past the context is read and not written); only the stores are predicated
     u32x2 c[kKV];
@@ -476,7 +485,7 @@ __global__ __launch_bounds__(256) void dequant_paged_list(DequantParams p,
 #pragma unroll
     for (int kv = 0; kv < kKV; ++kv) {
       c[kv] = __builtin_nontemporal_load(
-          reinterpret_cast<const u32x2*>(p.cache[kv] + e.blk * page_codes + (int64_t)u * 8));
+          reinterpret_cast<const u32x2*>(p.cache[kv] + e.blk * page_codes + code0));
       if constexpr (kMode == 1) sc[kv] = token_scale<kCS>(p.scale[kv], e.blk * page_rows + (u >> u8));
     }
 #pragma unroll
@@ -549,17 +558,23 @@ int launch(DequantParams p, void* workspace, int64_t workspace_bytes, hipStream_
   if (blocks > 0x7fffffffLL) return TMO_ERR_INVALID_ARGUMENT;
   const int u_shift = (p.head_dim % 16 == 0) ? ilog2_if_pow2(p.head_dim / 16) : -1;
   const int bs_shift = ilog2_if_pow2(p.block_size);
-  bool vec = u_shift >= 0 && bs_shift >= 0 &&
-             (int64_t)p.heads * p.block_size * (p.head_dim / 16) < (int64_t(1) << 30);
+  // part rows: whole 8-code chunks, 16 bytes of outputs or more (page-list path only)
+  int64_t row_units = 1;
+  while (row_units * 8 < p.head_dim) row_units *= 2;
+  const bool part = u_shift < 0 && p.head_dim % 8 == 0 && p.head_dim > 16;
+  bool vec = (u_shift >= 0 || part) && bs_shift >= 0 &&
+             (int64_t)p.heads * p.block_size * row_units < (int64_t(1) << 30);
+  const int codes_al = part ? 8 : 16;
   for (int kv = 0; kv < p.nkv && vec; ++kv) {
     vec = reinterpret_cast<uintptr_t>(p.out[kv]) % 16 == 0 &&
-          reinterpret_cast<uintptr_t>(p.cache[kv]) % 16 == 0 &&
+          reinterpret_cast<uintptr_t>(p.cache[kv]) % codes_al == 0 &&
           (p.out_st[kv] * kBytes) % 16 == 0 && (p.out_sh[kv] * kBytes) % 16 == 0 &&
           (p.mode == 1 || reinterpret_cast<uintptr_t>(p.scale[kv]) % 16 == 0);
   }
   const dim3 grid((unsigned)blocks), block(256);
-  if (!vec) return launch_kernel(dequant_paged_generic<Tag>, grid, block, stream, p);
-  p.u_shift = u_shift;
+  auto generic = [&]() { return launch_kernel(dequant_paged_generic<Tag>, grid, block, stream, p); };
+  if (!vec) return generic();
+  p.u_shift = part ? ilog2_if_pow2(row_units) - 1 : u_shift;
   p.bs_shift = bs_shift;
   p.h_shift = ilog2_if_pow2(p.heads);
   // page-list path: 256-unit items, a power of two of them per page, and a workspace.  Its
@@ -567,7 +582,7 @@ int launch(DequantParams p, void* workspace, int64_t workspace_bytes, hipStream_
   // rows, which gives one item per workgroup: with no context_seq_offset and non-negative
   // context lengths, page w of the flat list starts at output row >= (w - batch) *
   // block_size, so at most ceil(total_rows / BS) + batch pages write anything.
-  const int64_t page_units = (int64_t)p.heads * p.block_size * (p.head_dim / 8);
+  const int64_t page_units = (int64_t)p.heads * p.block_size * row_units;
   const int part_shift = page_units % 256 == 0 ? ilog2_if_pow2(page_units / 256) : -1;
   if (workspace != nullptr && part_shift >= 0 && part_shift <= 20 &&
       workspace_bytes >= list_workspace_bytes(p.batch, p.grid_blocks) &&
@@ -586,14 +601,22 @@ int launch(DequantParams p, void* workspace, int64_t workspace_bytes, hipStream_
     const int64_t cap = (0x7fffffffLL >> (part_shift + 3)) << 3;
     const int64_t want = std::min<int64_t>(bound, cap) << part_shift;
     const dim3 g((unsigned)want);
-    if (p.nkv == 2)
-      return p.mode == 1
-                 ? launch_kernel(dequant_paged_list<Tag, 1, 2, kCS>, g, block, stream, p, list, total)
-                 : launch_kernel(dequant_paged_list<Tag, 0, 2, kCS>, g, block, stream, p, list, total);
-    return p.mode == 1
-               ? launch_kernel(dequant_paged_list<Tag, 1, 1, kCS>, g, block, stream, p, list, total)
-               : launch_kernel(dequant_paged_list<Tag, 0, 1, kCS>, g, block, stream, p, list, total);
+    auto run = [&](auto mode, auto kvs) {
+      return launch_kernel(dequant_paged_list<Tag, decltype(mode)::value, decltype(kvs)::value, kCS>, g,
+                           block, stream, p, list, total);
+    };
+    auto with_kv = [&](auto mode) {
+      return p.nkv == 2 ? run(mode, std::integral_constant<int, 2>{})
+                        : run(mode, std::integral_constant<int, 1>{});
+    };
+    switch (p.mode | (part ? kPartRow : 0)) {
+      case 0: return with_kv(std::integral_constant<int, 0>{});
+      case 1: return with_kv(std::integral_constant<int, 1>{});
+      case kPartRow: return with_kv(std::integral_constant<int, kPartRow>{});
+      default: return with_kv(std::integral_constant<int, 1 | kPartRow>{});
+    }
   }
+  if (part) return generic();
   if (p.h_shift >= 0 && p.batch <= kPersistentMaxSeqs &&
       ((int64_t)p.heads << (bs_shift + u_shift)) % 256 == 0) {
     int device = 0, cus = 0;

@@ -686,6 +686,27 @@ def test_dequant_ignores_max_context_len(tmo, ref, dev, D, BS, H):
         _dequant_both(tmo, ref, dev, layout, caches, torch.bfloat16, 1, max_ctx=mctx)
 
 
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("D,BS,H", [(24, 16, 16), (40, 32, 2), (72, 16, 1), (80, 16, 4), (96, 16, 8),
+                                    (120, 32, 4), (144, 16, 2), (248, 16, 4), (264, 16, 2)])
+def test_dequant_part_rows(tmo, ref, dev, mode, D, BS, H):
+    """Head sizes whose 8-code chunks are no power of two on the page-list kernel: output types,
+    int8 and fp8 pages, fp32 and bf16 scales."""
+    layout, (kc, vc, ks, vs) = _small_layout(seed=D + BS + mode + H, D=D, BS=BS, NB=64, H=H)
+    if mode == 0:
+        g = torch.Generator().manual_seed(98)
+        ks = torch.rand(H, D, generator=g) * 0.05
+        vs = torch.rand(H, D, generator=g) * 0.05
+    caches = tuple(t.to(dev) for t in (kc, vc, ks, vs))
+    for dt in (torch.bfloat16, torch.float32):
+        _dequant_both(tmo, ref, dev, layout, caches, dt, mode)
+    fg = torch.Generator().manual_seed(97)
+    fp8 = tuple(W.fp8_codes(tuple(kc.shape), fg).to(dev) for _ in range(2))
+    bf = tuple(t.to(torch.bfloat16).to(dev) for t in (ks, vs))
+    _dequant_both(tmo, ref, dev, layout, fp8 + bf, torch.float16, mode)
+    _dequant_both(tmo, ref, dev, layout, fp8 + bf, torch.bfloat16, mode, with_v=False)
+
+
 def test_dequant_many_sequences(tmo, ref, dev):
     """More sequences than the persistent kernel keeps in LDS (per-page kernel), and a batch
     just below that limit (persistent kernel), with empty and single-token sequences."""
