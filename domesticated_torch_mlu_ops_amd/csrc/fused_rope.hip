@@ -138,19 +138,31 @@ __device__ __forceinline__ float rms_inverse_pow2(float ss, float eps) {
   return 1.0f / __builtin_sqrtf(a);
 }
 
+// RMS inverse of a row from its lanes' chunk sums; a part row's idle lanes add zeros, as in
+// fused_rope_generic, and the mean divides by its own length.
+template <int G, bool kPart>
+__device__ __forceinline__ float row_inverse(float acc, const FusedRopeParams& p, bool live) {
+  if constexpr (kPart) return rms_inverse(group_sum_f32<G>(live ? acc : 0.0f), p.head_dim, p.eps);
+  return rms_inverse_pow2<8 * G>(group_sum_f32<G>(acc), p.eps);
+}
+
 // Layernorm of a row held as G lanes x 8 values, D = 8 * G (reference _ops.py:3501-3504):
 // mean = RN(s1 / D), s1 the chunked sum of the values; d = RN(y - mean); var = RN(s2 / D), s2
 // the chunked sum of RN(d * d); inv = RN(1 / RN(sqrt(RN(var + eps))));
 // y = RN(RN(d * inv) * gamma) [+ beta, rounded].  D is a power of two, so the divisions by D
 // are exact products (rms_inverse_pow2).
-template <int G>
+// Part rows (kPart: d of the G lanes' 8 * G values, `live` false in the lanes past them) add zeros
+// for those lanes, as fused_rope_generic does, and divide by d.
+template <int G, bool kPart>
 __device__ __forceinline__ void layernorm8(float* y, const float* g, const float* b, bool has_beta,
-                                           float eps) {
+                                           float eps, int d, bool live) {
   constexpr int D = 8 * G;
   float s1 = y[0];
 #pragma unroll
   for (int e = 1; e < 8; ++e) s1 = s1 + y[e];
-  const float mean = group_sum_f32<G>(s1) * (1.0f / (float)D);
+  if (kPart && !live) s1 = 0.0f;
+  const float t1 = group_sum_f32<G>(s1);
+  const float mean = kPart ? t1 / (float)d : t1 * (1.0f / (float)D);
   float dv[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) dv[e] = y[e] - mean;
@@ -160,7 +172,9 @@ __device__ __forceinline__ void layernorm8(float* y, const float* g, const float
     const float sq = dv[e] * dv[e];
     s2 = s2 + sq;
   }
-  const float inv = rms_inverse_pow2<D>(group_sum_f32<G>(s2), eps);
+  if (kPart && !live) s2 = 0.0f;
+  const float t2 = group_sum_f32<G>(s2);
+  const float inv = kPart ? rms_inverse(t2, d, eps) : rms_inverse_pow2<D>(t2, eps);
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
     const float n = dv[e] * inv;
@@ -169,6 +183,7 @@ __device__ __forceinline__ void layernorm8(float* y, const float* g, const float
   }
 }
 
+constexpr int kPartRow = 128;      // flag beside a lane count: a row of fewer than G chunks
 constexpr int kDppRowRor8 = 0x128;  // rotate right by 8 lanes inside each 16-lane row
 
 #ifndef TMO_FUSED_ROPE_TOKEN_MAJOR
@@ -184,10 +199,14 @@ __device__ __forceinline__ void pack8(Tag, const float* f, u32x4& w) {
 // Vector path: head_dim = 8 * G (G a power of two <= 64), rope window on 8-element chunks.
 // kNorm (0 rmsnorm, 1 layernorm) is p.norm as a template argument, so the rmsnorm instance
 // carries no layernorm registers (p.norm is still what the generic kernel reads).
-template <class Tag, int G, int kNorm>
+template <class Tag, int GP, int kNorm>
 __global__ __launch_bounds__(256) void fused_rope_vec(FusedRopeParams p) {
+  constexpr int G = GP & (kPartRow - 1);
+  constexpr bool kPart = GP >= kPartRow;
   constexpr int kRows = 256 / G;
   const int lane = threadIdx.x & (G - 1);
+  const bool live_lane = !kPart || lane * 8 < p.head_dim;
+  const int at = kPart ? min(lane * 8, p.head_dim - 8) : lane * 8;  // the lane's chunk, clamped
   const int64_t row = (int64_t)blockIdx.x * kRows + threadIdx.x / G;
   const int64_t nrows = p.tokens * p.heads;
   // a group past the last row still runs the shuffles below (with its own lanes only) and
@@ -196,7 +215,7 @@ __global__ __launch_bounds__(256) void fused_rope_vec(FusedRopeParams p) {
   const int64_t t = live ? row / p.heads : 0;
   const int hh = live ? (int)(row - t * p.heads) : 0;
   const int kind = hh < p.hq ? 0 : (hh < p.hq + p.hk ? 1 : 2);  // q, k, v
-  char* xrow = static_cast<char*>(p.qkv) + (row * p.head_dim + lane * 8) * Tag::kBytes;
+  char* xrow = static_cast<char*>(p.qkv) + (row * p.head_dim + at) * Tag::kBytes;
 
   // ---- loads: x, then (q/k) gamma and the sin/cos of this lane's window chunk, slot
   u32x4 xw = {0u, 0u, 0u, 0u}, gw = {0u, 0u, 0u, 0u}, sw = {0u, 0u, 0u, 0u}, cw = {0u, 0u, 0u, 0u};
@@ -212,9 +231,9 @@ __global__ __launch_bounds__(256) void fused_rope_vec(FusedRopeParams p) {
     if (kind != 2) {
       const int64_t b = t / p.seq_len;
       pos = (int64_t)p.position[b] + (t - b * p.seq_len);
-      if (gamma) gw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(gamma) + lane * 16);
+      if (gamma) gw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(gamma) + at * 2);
       if (kind == 1 && kNorm == 1 && p.k_beta)
-        bw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.k_beta) + lane * 16);
+        bw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.k_beta) + at * 2);
       if (pos >= 0 && pos < p.table_rows && in_win) {
         const int64_t e = pos * p.table_stride + (lane - c0) * 8;
         sw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.sin_t) + e * Tag::kBytes);
@@ -236,7 +255,7 @@ __global__ __launch_bounds__(256) void fused_rope_vec(FusedRopeParams p) {
       const float sq = x[e] * x[e];
       acc = acc + sq;
     }
-    const float inv = rms_inverse_pow2<8 * G>(group_sum_f32<G>(acc), p.eps);
+    const float inv = row_inverse<G, kPart>(acc, p, live_lane);
     float g[8];
     unpack(Tag{}, gw, g);
 #pragma unroll
@@ -279,10 +298,10 @@ __global__ __launch_bounds__(256) void fused_rope_vec(FusedRopeParams p) {
       float g[8], bt[8];
       unpack(Tag{}, gw, g);
       unpack(Tag{}, bw, bt);
-      layernorm8<G>(y, g, bt, p.k_beta != nullptr, p.eps);
+      layernorm8<G, kPart>(y, g, bt, p.k_beta != nullptr, p.eps, p.head_dim, live_lane);
     }
   }
-  if (!live) return;
+  if (!live || (kPart && kind == 0 && !live_lane)) return;
   if (kind == 0) {
     u32x4 o;
     pack8(Tag{}, y, o);
@@ -296,6 +315,7 @@ __global__ __launch_bounds__(256) void fused_rope_vec(FusedRopeParams p) {
   int64_t page_row;
   if (!page_row_of(p, slot, h, page_row)) return;  // group-uniform
   if (p.scale_mode == 0) {
+    if (kPart && !live_lane) return;
     u32x4 o;
     pack8(Tag{}, y, o);
     *reinterpret_cast<u32x4*>(static_cast<char*>(cache_of(p, kv)) +
@@ -307,11 +327,12 @@ __global__ __launch_bounds__(256) void fused_rope_vec(FusedRopeParams p) {
     float m = 0.0f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) m = abs_max(m, y[e]);
+    if (kPart && !live_lane) m = 0.0f;
     const RowScale rs = make_row_scale(__uint_as_float(group_max_u32<G>(__float_as_uint(m))));
     encode_row<8>(y, rs, c);
     if (lane == 0) scale_of_kv(p, kv)[page_row] = rs.s;
   } else {
-    const float* sp = scale_of_kv(p, kv) + (int64_t)h * p.head_dim + lane * 8;
+    const float* sp = scale_of_kv(p, kv) + (int64_t)h * p.head_dim + at;
     float s[8], yr[8], q[8];
     bool fast = true;
 #pragma unroll
@@ -327,6 +348,7 @@ __global__ __launch_bounds__(256) void fused_rope_vec(FusedRopeParams p) {
       c[i] = pack_codes(code_bits(q[4 * i]), code_bits(q[4 * i + 1]), code_bits(q[4 * i + 2]),
                         code_bits(q[4 * i + 3]));
   }
+  if (kPart && !live_lane) return;
   u32x2 c2;
   c2[0] = c[0];
   c2[1] = c[1];
@@ -338,10 +360,14 @@ __global__ __launch_bounds__(256) void fused_rope_vec(FusedRopeParams p) {
 // its heads, kR rows per group, all kR rows loaded before the first is processed.  sin/cos
 // (with the rotation's sign folded in) are unpacked once per workgroup, both gammas loaded
 // once.  Same arithmetic, in the same order, as fused_rope_vec.
-template <class Tag, int G, int kR, int kNorm, int kThreads>
+template <class Tag, int GP, int kR, int kNorm, int kThreads>
 __global__ __launch_bounds__(kThreads) void fused_rope_tok(FusedRopeParams p) {
+  constexpr int G = GP & (kPartRow - 1);
+  constexpr bool kPart = GP >= kPartRow;
   constexpr int kGroups = kThreads / G;
   const int lane = threadIdx.x & (G - 1);
+  const bool live_lane = !kPart || lane * 8 < p.head_dim;
+  const int at = kPart ? min(lane * 8, p.head_dim - 8) : lane * 8;  // the lane's chunk, clamped
   const int grp = threadIdx.x / G;
   const int64_t t = blockIdx.x;
   const int64_t b = t / p.seq_len;  // workgroup-uniform (scalar)
@@ -352,7 +378,7 @@ __global__ __launch_bounds__(kThreads) void fused_rope_tok(FusedRopeParams p) {
   const bool rotate = pos >= 0 && pos < p.table_rows;  // workgroup-uniform
 
   // rows of this group: heads grp, grp + kGroups, ... (kR of them at most)
-  char* xbase = static_cast<char*>(p.qkv) + (t * p.heads * p.head_dim + lane * 8) * Tag::kBytes;
+  char* xbase = static_cast<char*>(p.qkv) + (t * p.heads * p.head_dim + at) * Tag::kBytes;
   // unconditional loads (a row past the last head re-reads the last head, in bounds, and is
   // not used): with the loads under a branch the compiler merged the array through register
   // copies that waited for each load before the next was issued
@@ -368,11 +394,11 @@ __global__ __launch_bounds__(kThreads) void fused_rope_tok(FusedRopeParams p) {
     sw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.sin_t) + e * Tag::kBytes);
     cw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.cos_t) + e * Tag::kBytes);
   }
-  kgw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.k_gamma) + lane * 16);
-  if (p.q_gamma) qgw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.q_gamma) + lane * 16);
+  kgw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.k_gamma) + at * 2);
+  if (p.q_gamma) qgw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.q_gamma) + at * 2);
   u32x4 kbw = {0u, 0u, 0u, 0u};
   if (kNorm == 1 && p.k_beta)
-    kbw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.k_beta) + lane * 16);
+    kbw = *reinterpret_cast<const u32x4*>(static_cast<const char*>(p.k_beta) + at * 2);
   // Every loaded register is used once here, before the first store: the stores count in the
   // same in-order memory counter as the loads, and a first use after a store (the rows after
   // the first, the gammas and sin/cos loaded under branches) made the compiler wait for that
@@ -409,7 +435,7 @@ __global__ __launch_bounds__(kThreads) void fused_rope_tok(FusedRopeParams p) {
           const float sq = y[e] * y[e];
           acc = acc + sq;
         }
-        const float inv = rms_inverse_pow2<8 * G>(group_sum_f32<G>(acc), p.eps);
+        const float inv = row_inverse<G, kPart>(acc, p, live_lane);
         float g[8];
         unpack(Tag{}, kind == 1 ? kgw : qgw, g);
 #pragma unroll
@@ -442,10 +468,11 @@ __global__ __launch_bounds__(kThreads) void fused_rope_tok(FusedRopeParams p) {
         float kg[8], kb[8];
         unpack(Tag{}, kgw, kg);
         unpack(Tag{}, kbw, kb);
-        layernorm8<G>(y, kg, kb, p.k_beta != nullptr, p.eps);
+        layernorm8<G, kPart>(y, kg, kb, p.k_beta != nullptr, p.eps, p.head_dim, live_lane);
       }
     }
     if (kind == 0) {
+      if (kPart && !live_lane) continue;
       u32x4 o;
       pack8(Tag{}, y, o);
       *reinterpret_cast<u32x4*>(xbase + (int64_t)hh * p.head_dim * Tag::kBytes) = o;
@@ -456,6 +483,7 @@ __global__ __launch_bounds__(kThreads) void fused_rope_tok(FusedRopeParams p) {
     int64_t page_row;
     page_row_of(p, slot, h, page_row);
     if (p.scale_mode == 0) {
+      if (kPart && !live_lane) continue;
       u32x4 o;
       pack8(Tag{}, y, o);
       *reinterpret_cast<u32x4*>(static_cast<char*>(cache_of(p, kv)) +
@@ -467,11 +495,12 @@ __global__ __launch_bounds__(kThreads) void fused_rope_tok(FusedRopeParams p) {
       float m = 0.0f;
 #pragma unroll
       for (int e = 0; e < 8; ++e) m = abs_max(m, y[e]);
+      if (kPart && !live_lane) m = 0.0f;
       const RowScale rs = make_row_scale(__uint_as_float(group_max_u32<G>(__float_as_uint(m))));
       encode_row<8>(y, rs, c);
       if (lane == 0) scale_of_kv(p, kv)[page_row] = rs.s;
     } else {
-      const float* sp = scale_of_kv(p, kv) + (int64_t)h * p.head_dim + lane * 8;
+      const float* sp = scale_of_kv(p, kv) + (int64_t)h * p.head_dim + at;
       float sc[8], yr[8], q[8];
       bool fast = true;
 #pragma unroll
@@ -487,6 +516,7 @@ __global__ __launch_bounds__(kThreads) void fused_rope_tok(FusedRopeParams p) {
         c[i] = pack_codes(code_bits(q[4 * i]), code_bits(q[4 * i + 1]), code_bits(q[4 * i + 2]),
                           code_bits(q[4 * i + 3]));
     }
+    if (kPart && !live_lane) continue;
     u32x2 c2;
     c2[0] = c[0];
     c2[1] = c[1];
@@ -656,7 +686,10 @@ int launch_tok(int r, hipStream_t stream, const FusedRopeParams& p) {
 template <class Tag, int kNorm>
 int launch(const FusedRopeParams& p, hipStream_t stream) {
   const int D = p.head_dim;
-  const int G = D / 8;
+  // lanes per row: D / 8, or for part rows (72..120 and 136..248 channels) the next power of two
+  int G = D / 8;
+  if (G > 8 && G < 32 && (G & (G - 1)) != 0) G = G < 16 ? 16 : 32;
+  const int gp = G * 8 == D ? G : G | kPartRow;
   auto al16 = [](const void* q) { return reinterpret_cast<uintptr_t>(q) % 16 == 0; };
   bool vec = D % 8 == 0 && G >= 1 && G <= kWave && (G & (G - 1)) == 0 &&
              p.rope_off % 8 == 0 && p.rope_dim % 16 == 0 && al16(p.qkv) && al16(p.k_gamma) && (!p.k_beta || al16(p.k_beta)) &&
@@ -670,7 +703,9 @@ int launch(const FusedRopeParams& p, hipStream_t stream) {
     const int64_t r = (p.heads + 256 / G - 1) / (256 / G);
     const int64_t r2 = (p.heads + 512 / G - 1) / (512 / G);
     if (r <= 3) {
-      switch (G) {
+      switch (gp) {
+        case 16 | kPartRow: return launch_tok<Tag, 16 | kPartRow, kNorm, 256, 3>((int)r, stream, p);
+        case 32 | kPartRow: return launch_tok<Tag, 32 | kPartRow, kNorm, 256, 3>((int)r, stream, p);
         case 1: return launch_tok<Tag, 1, kNorm, 256, 3>((int)r, stream, p);
         case 2: return launch_tok<Tag, 2, kNorm, 256, 3>((int)r, stream, p);
         case 4: return launch_tok<Tag, 4, kNorm, 256, 3>((int)r, stream, p);
@@ -681,7 +716,9 @@ int launch(const FusedRopeParams& p, hipStream_t stream) {
         default: break;
       }
     } else if (r2 <= kFusedRopeMaxRows) {
-      switch (G) {
+      switch (gp) {
+        case 16 | kPartRow: return launch_tok<Tag, 16 | kPartRow, kNorm, 512, kFusedRopeMaxRows, 2>((int)r2, stream, p);
+        case 32 | kPartRow: return launch_tok<Tag, 32 | kPartRow, kNorm, 512, kFusedRopeMaxRows, 2>((int)r2, stream, p);
         case 1: return launch_tok<Tag, 1, kNorm, 512, kFusedRopeMaxRows, 2>((int)r2, stream, p);
         case 2: return launch_tok<Tag, 2, kNorm, 512, kFusedRopeMaxRows, 2>((int)r2, stream, p);
         case 4: return launch_tok<Tag, 4, kNorm, 512, kFusedRopeMaxRows, 2>((int)r2, stream, p);
@@ -699,7 +736,9 @@ int launch(const FusedRopeParams& p, hipStream_t stream) {
   if (blocks > 0x7fffffffLL) return TMO_ERR_INVALID_ARGUMENT;
   const dim3 grid((unsigned)blocks), block(256);
   if (!vec) return launch_kernel(fused_rope_generic<Tag>, grid, block, stream, p);
-  switch (G) {
+  switch (gp) {
+    case 16 | kPartRow: return launch_kernel(fused_rope_vec<Tag, 16 | kPartRow, kNorm>, grid, block, stream, p);
+    case 32 | kPartRow: return launch_kernel(fused_rope_vec<Tag, 32 | kPartRow, kNorm>, grid, block, stream, p);
     case 1: return launch_kernel(fused_rope_vec<Tag, 1, kNorm>, grid, block, stream, p);
     case 2: return launch_kernel(fused_rope_vec<Tag, 2, kNorm>, grid, block, stream, p);
     case 4: return launch_kernel(fused_rope_vec<Tag, 4, kNorm>, grid, block, stream, p);

@@ -351,6 +351,20 @@ def check_fused_rope(tmo, ref, dev, name, case, with_q_gamma=True, off=0, api="r
                               f"{name} {n}")
 
 
+@pytest.mark.parametrize("mode", ["none", "dynamic", "static"])
+@pytest.mark.parametrize("norm_type", ["rmsnorm", "layernorm"])
+@pytest.mark.parametrize("D,rope,off,Hq,Hk", [(72, 64, 8, 8, 2), (80, 80, 0, 32, 8), (96, 96, 0, 4, 2),
+                                              (120, 32, 88, 6, 1), (136, 128, 0, 64, 8),
+                                              (248, 240, 8, 3, 3), (96, 64, 16, 200, 8)])
+def test_fused_rope_part_rows(tmo, ref, dev, D, rope, off, Hq, Hk, norm_type, mode):
+    """Head sizes that leave lanes of a row's group idle, on the token-major kernels (256 and 512
+    threads) and the row-major one (216 heads)."""
+    case = W.fused_rope_case(torch.bfloat16, mode, 23 + D, B=3, S=20, Hq=Hq, Hk=Hk, D=D, rope=rope)
+    beta = torch.linspace(-1.0, 1.0, D).to(torch.bfloat16) if norm_type == "layernorm" else None
+    check_fused_rope(tmo, ref, dev, f"part D={D} {norm_type} {mode}", case, True, off=off,
+                     api="fused_rope", norm_type=norm_type, k_beta=beta)
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("mode", ["none", "dynamic", "static"])
 @pytest.mark.parametrize("with_q_gamma", [True, False])
