@@ -210,32 +210,44 @@ struct SmoothLds {
 };
 
 // One row of 64 * kV 16-byte vectors (this lane's vectors lane + 64 * i in w) -> smoothed
-// int8 codes (RN(x * smooth) per element, no FMA) and the row scale.
+// int8 codes (RN(x * smooth) per element, no FMA) and the row scale.  Rows of more than 16 vectors
+// per lane keep the raw vectors only and smooth them again for the codes: the smoothed row would
+// take 8 registers per vector.
 template <class Tag, int kV, class SmoothAt>
 __device__ __forceinline__ void quant_row(const u32x4 (&w)[kV], SmoothAt sm, int8_t* orow,
                                              float* scale_out, int lane) {
   constexpr int kPer = Tag::kPerVec;
   constexpr int kSV = kPer / 4;
-  float v[kV][kPer];
+  constexpr bool kTwice = kV * kPer > 128;
+  float v[kTwice ? 1 : kV][kPer];
   float mx = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kV; ++i) {
-    unpack(Tag{}, w[i], v[i]);
+  auto smoothed = [&](int i, u32x4 raw, float* out) {
+    unpack(Tag{}, raw, out);
 #pragma unroll
     for (int q = 0; q < kSV; ++q) {
       const u32x4 sv = sm(i, q);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        v[i][4 * q + e] = v[i][4 * q + e] * __uint_as_float(sv[e]);
-        mx = abs_max(mx, v[i][4 * q + e]);
-      }
+      for (int e = 0; e < 4; ++e) out[4 * q + e] = out[4 * q + e] * __uint_as_float(sv[e]);
     }
+  };
+#pragma unroll
+  for (int i = 0; i < kV; ++i) {
+    float* x = v[kTwice ? 0 : i];
+    smoothed(i, w[i], x);
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) mx = abs_max(mx, x[e]);
   }
   const RowScale rs = make_row_scale(wave_max_uniform(mx));
 #pragma unroll
   for (int i = 0; i < kV; ++i) {
+    float* x = v[kTwice ? 0 : i];
+    if constexpr (kTwice) {
+      u32x4 raw = w[i];
+      asm volatile("" : "+v"(raw));  // or the compiler keeps the first pass's products
+      smoothed(i, raw, x);
+    }
     uint32_t c[kPer / 4];
-    encode_row<kPer>(v[i], rs, c);
+    encode_row<kPer>(x, rs, c);
     if constexpr (kPer == 8) {
       u32x2 c2;
       c2[0] = c[0];
@@ -359,10 +371,13 @@ __device__ __forceinline__ void sq_grp_row(const SqParams& p, u32x4* lds, int64_
 // From LDS the smooth row costs one staging per workgroup; read from L2 instead, every row
 // fetches its whole smooth row -- twice the row's own bytes, and twice its vector loads.
 // configs[3]-MoE on MI355X: 38.6 us with per-row L2 smooth reads (one wavefront per row,
-// index and group lookups serialised in front of the row loads), 34.0 us here.  Measured and
+// index and group lookups serialised in front of the row loads), 34.0 us here.  Expert rows of
+// 3584 / 5120 / 7168 / 14336 / 16384 channels (4099 tokens, top-2 of 64 experts): 19.0 / 29.9 /
+// 37.2 / 80.7 / 92.1 us with per-row reads, 17.1 / 22.7 / 30.8 / 73 / 83.9 us here.  Measured and
 // rejected: a fifth, staging-only wavefront per workgroup (37.0 us), 8 rows per workgroup
 // (35.8 us), a two-pass encoder that keeps only the raw row (60 VGPRs, 8 waves per SIMD,
-// 35.0 us).  A minimal kernel that only gathers and copies the same bytes takes 27.4 us.
+// 35.0 us; 10 and 14 vectors per lane: 23.6 and 31.8 us), and past 16 vectors 8 rows per
+// workgroup (16384 channels: 89.9 us).  A minimal kernel that only gathers and copies the same bytes takes 27.4 us.
 template <class Tag, int kV, int kW, bool kGroups, bool kGather>
 __global__ __launch_bounds__(64 * kW) void sq_grp(SqParams p) {
   constexpr int kSlot = kV * (Tag::kPerVec / 4) * kWave;
@@ -553,8 +568,17 @@ int launch_dense(const SqParams& p, hipStream_t stream) {
 // (two 16-byte loads and two 8-byte stores per thread per row) takes 17.8 us.  Rows mapped to
 // workgroups in contiguous blocks instead of strides, or loaded without the prefetch, were
 // 0.5-3 us slower.
-template <class Tag, int kV, bool kScalar, bool kChan>
+//
+// kVP is kV, plus kPartRow for rows of fewer than 256 * kV vectors: the threads past the row read
+// its last vector again in the last step, which leaves the maximum alone, and store nothing.
+// 4099 bf16 rows of 5120 / 7168 / 14336 / 16384 channels: 17.7 / 22.3 / 39.7 / 43.7 us on the
+// wavefront kernels (bounds checks on every vector; two wavefronts per row past 8192 channels),
+// 13.5 / 18.0 / 32.1 / 36.1 us here, 5.0-5.6 TB/s.
+constexpr int kPartRow = 64;  // flag beside a vector count
+template <class Tag, int kVP, bool kScalar, bool kChan>
 __global__ __launch_bounds__(256) void sq_dense_wg(SqParams p) {
+  constexpr int kV = kVP & (kPartRow - 1);
+  constexpr bool kPart = kVP >= kPartRow;
   constexpr int kPer = Tag::kPerVec;
   constexpr int kT = 256;
   __shared__ uint32_t red[2][4];
@@ -566,6 +590,13 @@ __global__ __launch_bounds__(256) void sq_dense_wg(SqParams p) {
   if (row >= rows) return;  // workgroup-uniform
   const int64_t row_bytes = p.row_stride * Tag::kBytes;
   const char* xb = static_cast<const char*>(p.x);
+  // vector i of this thread, and the last step's clamped to the row
+  const int nvec = (int)(p.channels / kPer);
+  const bool own_last = !kPart || tid + kT * (kV - 1) < nvec;
+  auto vec_of = [&](int i) -> int {
+    const int u = tid + kT * i;
+    return kPart && i == kV - 1 && !own_last ? nvec - 1 : u;
+  };
 
   // Offsets are masked rather than branched on: a branch let the compiler merge the two paths'
   // loads through register copies (and drop the non-temporal hint of one of them).
@@ -573,7 +604,7 @@ __global__ __launch_bounds__(256) void sq_dense_wg(SqParams p) {
     const int64_t mask = -(int64_t)real;
 #pragma unroll
     for (int i = 0; i < kV; ++i) {
-      const int64_t off = (r * row_bytes + (int64_t)(tid + kT * i) * 16) & mask;
+      const int64_t off = (r * row_bytes + (int64_t)vec_of(i) * 16) & mask;
       w[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(xb + off));
     }
   };
@@ -588,7 +619,7 @@ __global__ __launch_bounds__(256) void sq_dense_wg(SqParams p) {
   if constexpr (kChan) {
 #pragma unroll
     for (int i = 0; i < kV; ++i) {
-      const u32x4* sp = reinterpret_cast<const u32x4*>(p.smooth + (int64_t)(tid + kT * i) * kPer);
+      const u32x4* sp = reinterpret_cast<const u32x4*>(p.smooth + (int64_t)vec_of(i) * kPer);
 #pragma unroll
       for (int q = 0; q < kPer / 4; ++q) {
         const u32x4 s4 = sp[q];
@@ -650,6 +681,7 @@ __global__ __launch_bounds__(256) void sq_dense_wg(SqParams p) {
     for (int i = 0; i < kV; ++i) encode_row<kPer>(v[i], rs, keep + i * (kPer / 4));
 #pragma unroll
     for (int i = 0; i < kV; ++i) {
+      if (kPart && i == kV - 1 && !own_last) continue;
       const uint32_t off = (uint32_t)(tid + kT * i) * kPer;
       if constexpr (kPer == 8) {
         u32x2 c2;
@@ -682,7 +714,11 @@ int launch_dense_wg(const SqParams& p, hipStream_t stream) {
   if (hipGetDevice(&device) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess)
     return TMO_ERR_LAUNCH;
-  const int64_t blocks = std::min<int64_t>(p.dense_rows, (int64_t)cus * TMO_SQ_WG_ROW_PER_CU);
+  // Rows of five and more vectors per thread (133-211 registers with a smooth vector): two
+  // workgroups per CU, 36.1 us for 4099 rows of 16384 channels against 36.6-37.6 us with three
+  // and four; 5120 and 7168 channels are level.
+  const int64_t per_cu = (kV & (kPartRow - 1)) > 4 ? 2 : TMO_SQ_WG_ROW_PER_CU;
+  const int64_t blocks = std::min<int64_t>(p.dense_rows, (int64_t)cus * per_cu);
   const dim3 grid((unsigned)blocks), block(256);
   if (p.smooth && p.smooth_len != 1)
     return launch_kernel(sq_dense_wg<Tag, kV, false, true>, grid, block, stream, p);
@@ -742,9 +778,55 @@ int launch(const SqParams& p, hipStream_t stream) {
       (p.row_stride * Tag::kBytes) % 16 == 0 && reinterpret_cast<uintptr_t>(p.out) % 8 == 0 &&
       (!p.smooth || p.smooth_len == 1 || reinterpret_cast<uintptr_t>(p.smooth) % 16 == 0);
   const int64_t nvec = p.channels / kPer;
-  // One wavefront per row measured fastest (4096 channels: 20.4 us vs 23.0 us split over two);
-  // rows longer than 16 vectors per lane are split over two wavefronts rather than falling
-  // back to the scalar kernel.
+  const bool dense = !p.gather_index && !p.token_count;
+  // Dense rows of more than 128 vectors: a workgroup per row, up to the 8 vectors per thread that
+  // the registers hold twice over.  Shorter rows leave half of a workgroup's threads without one.
+  if (TMO_SQ_DENSE_WG && aligned && dense && nvec > 128 && nvec <= 8 * 256) {
+    switch ((nvec + 255) / 256 + (nvec % 256 ? kPartRow : 0)) {
+      case 1: return launch_dense_wg<Tag, 1>(p, stream);
+      case 2: return launch_dense_wg<Tag, 2>(p, stream);
+      case 3: return launch_dense_wg<Tag, 3>(p, stream);
+      case 4: return launch_dense_wg<Tag, 4>(p, stream);
+      case 5: return launch_dense_wg<Tag, 5>(p, stream);
+      case 6: return launch_dense_wg<Tag, 6>(p, stream);
+      case 7: return launch_dense_wg<Tag, 7>(p, stream);
+      case 8: return launch_dense_wg<Tag, 8>(p, stream);
+      case 1 + kPartRow: return launch_dense_wg<Tag, 1 + kPartRow>(p, stream);
+      case 2 + kPartRow: return launch_dense_wg<Tag, 2 + kPartRow>(p, stream);
+      case 3 + kPartRow: return launch_dense_wg<Tag, 3 + kPartRow>(p, stream);
+      case 4 + kPartRow: return launch_dense_wg<Tag, 4 + kPartRow>(p, stream);
+      case 5 + kPartRow: return launch_dense_wg<Tag, 5 + kPartRow>(p, stream);
+      case 6 + kPartRow: return launch_dense_wg<Tag, 6 + kPartRow>(p, stream);
+      case 7 + kPartRow: return launch_dense_wg<Tag, 7 + kPartRow>(p, stream);
+      default: return launch_dense_wg<Tag, 8 + kPartRow>(p, stream);
+    }
+  }
+  // Gathered / grouped rows with per-channel smooth rows: the LDS-staged kernel wherever the row
+  // is a whole number of 64-lane steps (every fourth past 16; 32 steps fill 64 KiB of LDS)
+  if (aligned && !dense && p.inner == 1 && p.smooth && p.channels > 1 &&
+      p.smooth_len == p.channels && nvec % kWave == 0) {
+    switch (nvec / kWave) {
+      case 1: return launch_grp<Tag, 1>(p, stream);
+      case 2: return launch_grp<Tag, 2>(p, stream);
+      case 3: return launch_grp<Tag, 3>(p, stream);
+      case 4: return launch_grp<Tag, 4>(p, stream);
+      case 5: return launch_grp<Tag, 5>(p, stream);
+      case 6: return launch_grp<Tag, 6>(p, stream);
+      case 7: return launch_grp<Tag, 7>(p, stream);
+      case 8: return launch_grp<Tag, 8>(p, stream);
+      case 10: return launch_grp<Tag, 10>(p, stream);
+      case 12: return launch_grp<Tag, 12>(p, stream);
+      case 14: return launch_grp<Tag, 14>(p, stream);
+      case 16: return launch_grp<Tag, 16>(p, stream);
+      case 20: return launch_grp<Tag, 20>(p, stream);
+      case 24: return launch_grp<Tag, 24>(p, stream);
+      case 28: return launch_grp<Tag, 28>(p, stream);
+      case 32: return launch_grp<Tag, 32>(p, stream);
+      default: break;
+    }
+  }
+  // Rows longer than 16 vectors per lane are split over two wavefronts rather than falling back
+  // to the scalar kernel.
   constexpr int kW = TMO_SQ_WAVES_PER_ROW;
   const bool split = kW > 1 && nvec > 16 * kWave;
   const int64_t per_lane = (nvec + kWave * (split ? kW : 1) - 1) / (kWave * (split ? kW : 1));
@@ -754,31 +836,10 @@ int launch(const SqParams& p, hipStream_t stream) {
     if (p.gather_index) return launch_vec<Tag, false, kW>(p, per_lane, stream);
     return launch_vec<Tag, true, kW>(p, per_lane, stream);
   }
-  if (TMO_SQ_DENSE_WG && !p.gather_index && !p.token_count && nvec % 256 == 0) {
-    switch (nvec / 256) {
-      case 1: return launch_dense_wg<Tag, 1>(p, stream);
-      case 2: return launch_dense_wg<Tag, 2>(p, stream);
-      case 4: return launch_dense_wg<Tag, 4>(p, stream);
-      default: break;
-    }
-  }
-  if (!p.gather_index && !p.token_count && nvec % kWave == 0) {
+  if (dense && nvec % kWave == 0) {
     switch (nvec / kWave) {
       case 1: return launch_dense<Tag, 1>(p, stream);
       case 2: return launch_dense<Tag, 2>(p, stream);
-      case 4: return launch_dense<Tag, 4>(p, stream);
-      case 8: return launch_dense<Tag, 8>(p, stream);
-      case 16: return launch_dense<Tag, 16>(p, stream);
-      default: break;
-    }
-  }
-  if ((p.gather_index || p.token_count) && p.inner == 1 && p.smooth && p.channels > 1 &&
-      p.smooth_len == p.channels && nvec % kWave == 0) {
-    switch (nvec / kWave) {
-      case 1: return launch_grp<Tag, 1>(p, stream);
-      case 2: return launch_grp<Tag, 2>(p, stream);
-      case 4: return launch_grp<Tag, 4>(p, stream);
-      case 8: return launch_grp<Tag, 8>(p, stream);
       default: break;
     }
   }

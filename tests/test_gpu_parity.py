@@ -988,6 +988,36 @@ def test_smooth_quant_grouped_rows(tmo, ref, dev, dtype, C):
                                               0.5 + torch.rand(C, generator=g), None, gi))
 
 
+@pytest.mark.parametrize("dtype,C", [
+    (torch.bfloat16, 1032), (torch.bfloat16, 3584), (torch.bfloat16, 5128), (torch.bfloat16, 7168),
+    (torch.bfloat16, 14336), (torch.bfloat16, 16376), (torch.float16, 10240), (torch.float32, 4092),
+    (torch.float32, 8192)])
+def test_smooth_quant_wide_rows(tmo, ref, dev, dtype, C):
+    """Widths between the whole 256-thread steps (one vector past a step, one short of the largest
+    width) and the widest rows, dense with per-channel, scalar and no smooth, 3-D and as a column
+    slice, gathered and grouped; more rows than one launch has workgroups."""
+    g = torch.Generator().manual_seed(C + 13)
+    n0 = 1100
+    x = (torch.randn(n0, C, generator=g) * torch.logspace(-2, 2, n0)[:, None]).to(dtype)
+    x[7] = 0
+    x[11, : C - 1] = 0                     # the maximum in the row's last element
+    sm = 0.5 + torch.rand(C, generator=g)
+    _sq_both(tmo, ref, dev, W.SmoothQuantCase(f"channel {dtype} C={C}", x, sm))
+    few = x[:60]
+    _sq_both(tmo, ref, dev, W.SmoothQuantCase("scalar", few, torch.tensor([0.75])))
+    _sq_both(tmo, ref, dev, W.SmoothQuantCase("none", few, torch.ones(C)), smooth=False)
+    _sq_both(tmo, ref, dev, W.SmoothQuantCase("3d", few.view(20, 3, C), sm))
+    wide = torch.full((60, C + 64), 1e4, dtype=dtype)   # columns past the slice must not count
+    wide[:, :C] = few
+    _sq_both(tmo, ref, dev, W.SmoothQuantCase("slice", few, sm), x_dev=wide.to(dev)[:, :C])
+    tc = torch.tensor([3, 0, 17, 1, 2, 40, 5], dtype=torch.int32)
+    gi = torch.randint(0, n0, (int(tc.sum()) + 3,), generator=g).to(torch.int32)
+    gi[5] = n0
+    _sq_both(tmo, ref, dev, W.SmoothQuantCase("groups", x, 0.5 + torch.rand(7, C, generator=g),
+                                              tc, gi))
+    _sq_both(tmo, ref, dev, W.SmoothQuantCase("gather", x, sm, None, gi))
+
+
 def test_public_wrappers(tmo, ref, dev):
     """scaled_quantize and the per_token_smooth_quantize alias return what moe_quantize does."""
     case = W.cfg4()
