@@ -196,7 +196,9 @@ __device__ __forceinline__ void pack8(Tag, const float* f, u32x4& w) {
   for (int i = 0; i < 4; ++i) w[i] = pack2(Tag{}, f[2 * i], f[2 * i + 1]);
 }
 
-// Vector path: head_dim = 8 * G (G a power of two <= 64), rope window on 8-element chunks.
+// Vector path: head_dim = 8 * G (G a power of two <= 64), rope window on 8-element chunks; with
+// kPartRow, fewer than G chunks (4 x 4096 tokens, 32 + 8 heads x 96: 482 us on the generic kernel,
+// 76 us here).
 // kNorm (0 rmsnorm, 1 layernorm) is p.norm as a template argument, so the rmsnorm instance
 // carries no layernorm registers (p.norm is still what the generic kernel reads).
 template <class Tag, int GP, int kNorm>
