@@ -85,11 +85,12 @@ __global__ __launch_bounds__(256 * kCB, 2) void attn_latent(AttnParams p) {
   const int col = lane & 15, grp = lane >> 4;
   const int chq = wave & 3;           // quarter of the value channels, and:
   const int st_tile = chq % kST, st_half = chq / kST;  // score tile, part of its channels
-  const int64_t i = blockIdx.z;
-  const int hk = blockIdx.y;
-  const int cbg = (int)(blockIdx.x / (unsigned)p.splits);  // group of kCB column blocks
-  const int split = (int)blockIdx.x - cbg * p.splits;
-  const Seq sq = seq_of(p, i);
+  Work wk;
+  if (!work_of(p, (p.ncb + kCB - 1) / kCB, wk)) return;
+  const int64_t i = wk.i;
+  const int hk = wk.hk, split = wk.split;
+  const int cbg = wk.cb;  // group of kCB column blocks
+  const Seq sq = wk.sq;
   const Range rg = token_range(p, sq, split);
   if (p.splits > 1 && rg.begin >= rg.end) return;  // an empty split writes no partial
   const int c = (cbg * kCB + (wave >> 2)) * 16 + col;
@@ -366,7 +367,7 @@ __global__ __launch_bounds__(256 * kCB, 2) void attn_latent(AttnParams p) {
 
 template <bool kF16, int kCB>
 int launch(const AttnParams& p, hipStream_t st) {
-  const dim3 grid((unsigned)(p.splits * ((p.ncb + kCB - 1) / kCB)), (unsigned)p.Hkv, (unsigned)p.B);
+  const dim3 grid = attn_grid(p, (p.ncb + kCB - 1) / kCB);
   const dim3 block(256 * kCB);
   return p.mask ? launch_kernel(attn_latent<kF16, kCB, true>, grid, block, st, p)
                 : launch_kernel(attn_latent<kF16, kCB, false>, grid, block, st, p);

@@ -41,8 +41,10 @@
 //     end.  The sink joins the denominator when the output is written.
 // The four wavefronts combine through LDS; with more than one split per (sequence, KV head)
 // the partials (max, sum, normalised row) go to a caller-provided workspace and a combine
-// kernel merges them.  A generic kernel (one wavefront per (query token, query head), VALU)
-// serves every other shape, dtype and scale layout.
+// kernel merges them.  K rows of 576 channels whose first 512 are the value row (attn_latent.hip)
+// and many query columns per KV head or head sizes 80 and 96 (attn_chunk.hip) have kernels of
+// their own.  A generic kernel (one wavefront per (query token, query head), VALU) serves every
+// other shape, dtype and scale layout.
 #include "attn_common.h"
 
 namespace tmo {
@@ -167,18 +169,15 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
   if (p.q_vec) {  // 16-byte aligned q rows of a 2-byte type: kDC / 8 vectors per lane
     constexpr int kQV = kDC / 8;
     u32x4 qraw[kQV];
-    const u32x4* qp = reinterpret_cast<const u32x4*>(
-        static_cast<const uint16_t*>(p.q) + i * p.q_sb + qrow * p.q_ss + (int64_t)hq * p.q_sh +
-        grp * kDC);
+    const uint16_t* qp = static_cast<const uint16_t*>(p.q) + i * p.q_sb + qrow * p.q_ss +
+                         (int64_t)hq * p.q_sh;
 #pragma unroll
     for (int v = 0; v < kQV; ++v) qraw[v] = qvalid ? qp[v] : u32x4{0u, 0u, 0u, 0u};
     // per-channel key scales of the lane's channels, raw: fp32 (4 per vector) or bf16 (8)
     constexpr int kCS = kQuant ? (kSB ? kDC / 8 : kDC / 4) : 1;
     u32x4 kcs[kCS];
     if (kQuant && p.smode == 2) {
-      const int64_t e0 = (int64_t)hk * kD + grp * kDC;
-      const u32x4* sp = kSB ? reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(p.ks) + e0)
-                            : reinterpret_cast<const u32x4*>(static_cast<const float*>(p.ks) + e0);
+      const int64_t e0 = (int64_t)hk * kD;
 #pragma unroll
       for (int v = 0; v < kCS; ++v) kcs[v] = sp[v];
     }
@@ -939,7 +938,7 @@ int launch_combine(const AttnParams& p, hipStream_t st) {
 
 template <int kD, int kKind, bool kSB>
 int launch_mfma_d(const AttnParams& p, bool qlo, hipStream_t st) {
-  const dim3 grid((unsigned)(p.splits * p.ncb), (unsigned)p.Hkv, (unsigned)p.B), block(256);
+  const dim3 grid = attn_grid(p, p.ncb), block(256);
   int rc;
   if (p.mask)
     rc = qlo ? launch_kernel(attn_mfma<kD, kKind, true, kSB, true>, grid, block, st, p)
@@ -1233,6 +1232,9 @@ extern "C" int tmo_hip_cached_kv_attn(
   if (cache_dtype == TMO_DTYPE_I8)
     return p.s_bf16 ? launch_mfma<0, true>(p, qlo, st) : launch_mfma<0, false>(p, qlo, st);
   if (cache_dtype == TMO_DTYPE_F8E4M3)
+  // Packed numbering for up to 64 sequences, one lane each; one sequence has nothing to even out
+  p.packed = p.splits > 1 && batch > 1 && batch <= kWave && p.split_tokens < (1LL << 31) &&
+             (int64_t)p.splits * p.ncb * num_kv_heads * batch < (1LL << 24);
     return p.s_bf16 ? launch_mfma<3, true>(p, qlo, st) : launch_mfma<3, false>(p, qlo, st);
   if (int4)
     return p.s_bf16 ? launch_mfma<4, true>(p, qlo, st) : launch_mfma<4, false>(p, qlo, st);
@@ -1243,6 +1245,7 @@ extern "C" int tmo_hip_cached_kv_attn(
 extern "C" int tmo_hip_single_query_cached_kv_attn(
     const void* q, int64_t q_stride_seq, int64_t q_stride_head, const void* k_cache,
     const void* v_cache, const float* k_scale, const float* v_scale, int scale_mode,
+    p.packed = 0;
     const int32_t* block_tables, int64_t max_blocks, const int32_t* context_lens,
     const float* alibi_slopes, void* out, int64_t out_stride_seq, int64_t out_stride_head,
     float* lse, int64_t lse_stride_seq, int64_t lse_stride_head, int64_t batch,
