@@ -20,9 +20,9 @@
 // wavefronts owns one (sequence, KV head, split, column block) and its wavefronts take every
 // fourth 16-token tile.  Per tile:
 //   * S^T = K Q^T with v_mfma_f32_16x16x16 (tokens are the rows, the block's query columns the
-//     columns, zero-padded to 16): lane (t = l % 16, c = l / 16) holds token t's channels
-//     [c D/4, (c + 1) D/4), so the K tile is read as contiguous row pieces, and MFMA m takes
-//     channels c D/4 + 4m .. + 3 of every lane group (a permutation of the reduction order).
+//     columns, zero-padded to 16): lane (t = l % 16, c = l / 16) holds every fourth 16-byte
+//     vector of token t's row from vector c on, and MFMA m takes channels 4m .. + 3 of every
+//     lane group's own (a permutation of the reduction order).
 //     Int8 codes enter as exact f16 values 1152 + code (two byte permutes per four codes) against
 //     a power-of-two scaled f16 q, and 1152 * sum(q) is subtracted from the fp32 result; the
 //     per-token scale and softmax_scale * log2(e) then multiply it.  Int4 codes enter as
@@ -77,6 +77,13 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
   using M = Mfma<kF16>;
   using V4 = typename M::V4;
   constexpr int kDC = kD / 4;       // channels per lane group in the K layout
+  // K channels per vector load of a lane.  The lane groups' vectors alternate along the row, so
+  // one load of the wavefront covers 64 contiguous bytes of each token: channel c of a lane's kDC
+  // is channel k_channel(c) of the row.  With one contiguous run of the row per lane, the loads of
+  // rows longer than 64 bytes strode over it, a quarter (bf16, 128 channels) of each 64-byte line
+  // at a time: 8 sequences of 128..4096 keys, 32 / 8 heads x 128 bf16: 39.5 -> 34.0 us, 32
+  // sequences of 512..4096 keys: 95 -> 77 us (int8 rows of 128 bytes: level).
+  constexpr int kKV = (kKind == 1 || kKind == 2) ? 8 : kKind == 4 ? (kDC < 32 ? kDC : 32) : 16;
   constexpr int kDV = kD / 16;      // channels per lane in the V layout
   constexpr int kQK = kD / 16;      // QK MFMAs per tile
   constexpr int kEs = kQuant ? 1 : 2;  // cache element bytes
@@ -88,11 +95,13 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
   const int col = lane & 15;        // query column within the block / token row
   const int grp = lane >> 4;        // lane group c
-  const int64_t i = blockIdx.z;
-  const int hk = blockIdx.y;
-  const int cb = (int)(blockIdx.x / (unsigned)p.splits);   // column block
-  const int split = (int)blockIdx.x - cb * p.splits;
-  const Seq sq = seq_of(p, i);
+  auto k_channel = [&](int c) -> int { return (c / kKV * 4 + grp) * kKV + c % kKV; };
+  Work wk;
+  if (!work_of(p, p.ncb, wk)) return;
+  const int64_t i = wk.i;
+  const int hk = wk.hk, split = wk.split;
+  const int cb = wk.cb;  // column block
+  const Seq sq = wk.sq;
   const Range rg = token_range(p, sq, split);
   // An empty split (past the sequence's keys) writes no partial; the combine skips it.  With
   // one split the (zero) output and lse are still written below.
@@ -172,14 +181,20 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
     const uint16_t* qp = static_cast<const uint16_t*>(p.q) + i * p.q_sb + qrow * p.q_ss +
                          (int64_t)hq * p.q_sh;
 #pragma unroll
-    for (int v = 0; v < kQV; ++v) qraw[v] = qvalid ? qp[v] : u32x4{0u, 0u, 0u, 0u};
+    for (int v = 0; v < kQV; ++v)
+      qraw[v] = qvalid ? *reinterpret_cast<const u32x4*>(qp + k_channel(8 * v))
+                       : u32x4{0u, 0u, 0u, 0u};
     // per-channel key scales of the lane's channels, raw: fp32 (4 per vector) or bf16 (8)
     constexpr int kCS = kQuant ? (kSB ? kDC / 8 : kDC / 4) : 1;
     u32x4 kcs[kCS];
     if (kQuant && p.smode == 2) {
       const int64_t e0 = (int64_t)hk * kD;
 #pragma unroll
-      for (int v = 0; v < kCS; ++v) kcs[v] = sp[v];
+      for (int v = 0; v < kCS; ++v)
+        kcs[v] = kSB ? *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(p.ks) + e0 +
+                                                       k_channel(8 * v))
+                     : *reinterpret_cast<const u32x4*>(static_cast<const float*>(p.ks) + e0 +
+                                                       k_channel(4 * v));
     }
     refill();
     const bool bf = p.q_dtype == TMO_DTYPE_BF16;
@@ -208,7 +223,7 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
     for (int m = 0; m < kQK; ++m) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int d = grp * kDC + qk_channel(kInt4, m, e);
+        const int d = k_channel(qk_channel(kInt4, m, e));
         float x = qvalid ? load_q(p, i * p.q_sb + qrow * p.q_ss + (int64_t)hq * p.q_sh + d) : 0.0f;
         if (kQuant && p.qs_mode == 3 && qvalid)  // group-wise q scales (kQLo holds the rest)
           x *= q_group_scale(p, i * p.qs_sb + qrow * p.qs_ss + (int64_t)hq * p.qs_sh, d);
@@ -283,7 +298,8 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
   const int64_t page_bytes = (int64_t)p.BS * kKRow;         // one head's page
   // per-lane offsets inside a 16-row piece of a page: K token `col`, channels grp * kDC ..;
   // V tokens 4 grp .. + 3, channels col * kDV ..
-  const int32_t k_lane = col * kKRow + grp * (kInt4 ? kDC / 2 : kDC * kEs);
+  constexpr int kKStep = kInt4 ? kKV / 2 : kKV * kEs;       // bytes of one vector
+  const int32_t k_lane = col * kKRow + grp * kKStep;
   const int32_t v_lane = kVRows * grp * kVRow + col * kDV * (kInt4 ? 1 : kEs);
   constexpr int kKW = kInt4 ? kDC / 8 : kDC * kEs / 4;      // dwords per lane
   constexpr int kVW = kInt4 ? kDV / 4 : kDV * kEs / 4;
@@ -310,7 +326,7 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
     if constexpr (kKW >= 4) {
 #pragma unroll
       for (int u = 0; u < kKW / 4; ++u) {
-        const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(krow) + u);
+        const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(krow) + 4 * u);
 #pragma unroll
         for (int e = 0; e < 4; ++e) r.kw[4 * u + e] = w[e];
       }
@@ -1216,6 +1232,9 @@ extern "C" int tmo_hip_cached_kv_attn(
   int64_t per = (max_context_len + splits - 1) / splits;
   per = latent ? (per + 31) / 32 * 32 : (per + 63) / 64 * 64;
   p.split_tokens = per > 0 ? per : 64;
+  // Packed numbering for up to 64 sequences, one lane each; one sequence has nothing to even out
+  p.packed = p.splits > 1 && batch > 1 && batch <= kWave && p.split_tokens < (1LL << 31) &&
+             (int64_t)p.splits * p.ncb * num_kv_heads * batch < (1LL << 24);
   if (latent) {
     const int rc = launch_attn_latent(p, st);
     return rc != TMO_OK || p.splits == 1 ? rc : launch_combine(p, st);
@@ -1226,15 +1245,13 @@ extern "C" int tmo_hip_cached_kv_attn(
   const bool qlo = scale_mode == 2 || p.qs_mode == 3;
   if (chunk) {
     p.lone = 1;
+    p.packed = 0;
     const int rc = launch_attn_chunk(p, qlo, st);
     return rc != TMO_OK || p.splits == 1 ? rc : launch_combine(p, st);
   }
   if (cache_dtype == TMO_DTYPE_I8)
     return p.s_bf16 ? launch_mfma<0, true>(p, qlo, st) : launch_mfma<0, false>(p, qlo, st);
   if (cache_dtype == TMO_DTYPE_F8E4M3)
-  // Packed numbering for up to 64 sequences, one lane each; one sequence has nothing to even out
-  p.packed = p.splits > 1 && batch > 1 && batch <= kWave && p.split_tokens < (1LL << 31) &&
-             (int64_t)p.splits * p.ncb * num_kv_heads * batch < (1LL << 24);
     return p.s_bf16 ? launch_mfma<3, true>(p, qlo, st) : launch_mfma<3, false>(p, qlo, st);
   if (int4)
     return p.s_bf16 ? launch_mfma<4, true>(p, qlo, st) : launch_mfma<4, false>(p, qlo, st);
@@ -1245,7 +1262,6 @@ extern "C" int tmo_hip_cached_kv_attn(
 extern "C" int tmo_hip_single_query_cached_kv_attn(
     const void* q, int64_t q_stride_seq, int64_t q_stride_head, const void* k_cache,
     const void* v_cache, const float* k_scale, const float* v_scale, int scale_mode,
-    p.packed = 0;
     const int32_t* block_tables, int64_t max_blocks, const int32_t* context_lens,
     const float* alibi_slopes, void* out, int64_t out_stride_seq, int64_t out_stride_head,
     float* lse, int64_t lse_stride_seq, int64_t lse_stride_head, int64_t batch,

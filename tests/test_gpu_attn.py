@@ -823,3 +823,25 @@ def test_attn_many_columns_quantised_q_and_sparse_tables(tmo, ref, dev):
     q = _q_codes(torch.int8, (3, 20, 8, 128), 172)
     for form in ("token", "group"):
         run_attn_mq(tmo, ref, dev, case, q, q_scale=_q_scale(form, (3, 20, 8), 173))
+
+
+@pytest.mark.parametrize("B", [1, 2, 64, 65])
+@pytest.mark.parametrize("kv,D", [("plain", 64), ("int8_channel", 128), ("int4_token", 256)])
+def test_attn_ragged_over_splits(tmo, ref, dev, kv, D, B):
+    """Ragged sequences over several splits, numbered live workgroups first (2 to 64 sequences) or
+    by the grid (1, 65): empty sequences first and last, one key, the edges of a split, the
+    maximum; one and two column blocks; a window; ragged query counts with a sequence of none."""
+    case = W.attn_case(torch.bfloat16, 180 + B, kv=kv, B=B, Hq=16, Hkv=2, D=D, BS=16, NB=46 * B,
+                       max_ctx=730)
+    if B > 1:
+        edges = [0, 730, 1, 256, 257, 255, 512, 513, 729]
+        lens = [edges[i % 9] for i in range(B)]
+        lens[-1] = 730 if B == 2 else 0
+        case.context_lens = torch.tensor(lens, dtype=torch.int32)
+    for S in (1, 3):
+        q = W.attn_queries(torch.bfloat16, 181, B=B, Hq=16, D=D, S=S)
+        run_attn_mq(tmo, ref, dev, case, q)
+        run_attn_mq(tmo, ref, dev, case, q, window=300, max_ctx=600)
+    q3, cu = W.attn_queries(torch.bfloat16, 182, B=B, Hq=16, D=D,
+                            counts=[(i + 1) % 4 for i in range(B)])
+    run_attn_mq(tmo, ref, dev, case, q3, cu=cu, max_seq_q=3)
