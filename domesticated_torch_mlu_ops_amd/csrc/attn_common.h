@@ -3,6 +3,7 @@
 // sequence and key-range rules, the softmax's last step, and the MFMA operand conversions.
 #pragma once
 
+#include "attn_rules.h"
 #include "tmo_device.h"
 
 namespace tmo {

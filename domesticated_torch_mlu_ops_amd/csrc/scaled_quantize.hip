@@ -210,44 +210,32 @@ struct SmoothLds {
 };
 
 // One row of 64 * kV 16-byte vectors (this lane's vectors lane + 64 * i in w) -> smoothed
-// int8 codes (RN(x * smooth) per element, no FMA) and the row scale.  Rows of more than 16 vectors
-// per lane keep the raw vectors only and smooth them again for the codes: the smoothed row would
-// take 8 registers per vector.
+// int8 codes (RN(x * smooth) per element, no FMA) and the row scale.
 template <class Tag, int kV, class SmoothAt>
 __device__ __forceinline__ void quant_row(const u32x4 (&w)[kV], SmoothAt sm, int8_t* orow,
                                              float* scale_out, int lane) {
   constexpr int kPer = Tag::kPerVec;
   constexpr int kSV = kPer / 4;
-  constexpr bool kTwice = kV * kPer > 128;
-  float v[kTwice ? 1 : kV][kPer];
+  float v[kV][kPer];
   float mx = 0.0f;
-  auto smoothed = [&](int i, u32x4 raw, float* out) {
-    unpack(Tag{}, raw, out);
+#pragma unroll
+  for (int i = 0; i < kV; ++i) {
+    unpack(Tag{}, w[i], v[i]);
 #pragma unroll
     for (int q = 0; q < kSV; ++q) {
       const u32x4 sv = sm(i, q);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) out[4 * q + e] = out[4 * q + e] * __uint_as_float(sv[e]);
+      for (int e = 0; e < 4; ++e) {
+        v[i][4 * q + e] = v[i][4 * q + e] * __uint_as_float(sv[e]);
+        mx = abs_max(mx, v[i][4 * q + e]);
+      }
     }
-  };
-#pragma unroll
-  for (int i = 0; i < kV; ++i) {
-    float* x = v[kTwice ? 0 : i];
-    smoothed(i, w[i], x);
-#pragma unroll
-    for (int e = 0; e < kPer; ++e) mx = abs_max(mx, x[e]);
   }
   const RowScale rs = make_row_scale(wave_max_uniform(mx));
 #pragma unroll
   for (int i = 0; i < kV; ++i) {
-    float* x = v[kTwice ? 0 : i];
-    if constexpr (kTwice) {
-      u32x4 raw = w[i];
-      asm volatile("" : "+v"(raw));  // or the compiler keeps the first pass's products
-      smoothed(i, raw, x);
-    }
     uint32_t c[kPer / 4];
-    encode_row<kPer>(x, rs, c);
+    encode_row<kPer>(v[i], rs, c);
     if constexpr (kPer == 8) {
       u32x2 c2;
       c2[0] = c[0];
@@ -372,12 +360,11 @@ __device__ __forceinline__ void sq_grp_row(const SqParams& p, u32x4* lds, int64_
 // fetches its whole smooth row -- twice the row's own bytes, and twice its vector loads.
 // configs[3]-MoE on MI355X: 38.6 us with per-row L2 smooth reads (one wavefront per row,
 // index and group lookups serialised in front of the row loads), 34.0 us here.  Expert rows of
-// 3584 / 5120 / 7168 / 14336 / 16384 channels (4099 tokens, top-2 of 64 experts): 19.0 / 29.9 /
-// 37.2 / 80.7 / 92.1 us with per-row reads, 17.1 / 22.7 / 30.8 / 73 / 83.9 us here.  Measured and
+// 3584 / 5120 / 7168 channels (4099 tokens, top-2 of 64 experts): 19.0 / 29.9 / 37.2 us with
+// per-row reads, 17.1 / 22.7 / 30.8 us here.  Measured and
 // rejected: a fifth, staging-only wavefront per workgroup (37.0 us), 8 rows per workgroup
 // (35.8 us), a two-pass encoder that keeps only the raw row (60 VGPRs, 8 waves per SIMD,
-// 35.0 us; 10 and 14 vectors per lane: 23.6 and 31.8 us), and past 16 vectors 8 rows per
-// workgroup (16384 channels: 89.9 us).  A minimal kernel that only gathers and copies the same bytes takes 27.4 us.
+// 35.0 us; 10 and 14 vectors per lane: 23.6 and 31.8 us).  A minimal kernel that only gathers and copies the same bytes takes 27.4 us.
 template <class Tag, int kV, int kW, bool kGroups, bool kGather>
 __global__ __launch_bounds__(64 * kW) void sq_grp(SqParams p) {
   constexpr int kSlot = kV * (Tag::kPerVec / 4) * kWave;
@@ -802,7 +789,9 @@ int launch(const SqParams& p, hipStream_t stream) {
     }
   }
   // Gathered / grouped rows with per-channel smooth rows: the LDS-staged kernel wherever the row
-  // is a whole number of 64-lane steps (every fourth past 16; 32 steps fill 64 KiB of LDS)
+  // is a whole number of 64-lane steps, up to 16.  Past those a row is split over two wavefronts
+  // below: staged, 14336 channels took 45.3 us for 2400 tokens (43.5 there) and 74 us for 4099
+  // (80.7), and 16.1 us for 300 (12.7).
   if (aligned && !dense && p.inner == 1 && p.smooth && p.channels > 1 &&
       p.smooth_len == p.channels && nvec % kWave == 0) {
     switch (nvec / kWave) {
@@ -818,10 +807,6 @@ int launch(const SqParams& p, hipStream_t stream) {
       case 12: return launch_grp<Tag, 12>(p, stream);
       case 14: return launch_grp<Tag, 14>(p, stream);
       case 16: return launch_grp<Tag, 16>(p, stream);
-      case 20: return launch_grp<Tag, 20>(p, stream);
-      case 24: return launch_grp<Tag, 24>(p, stream);
-      case 28: return launch_grp<Tag, 28>(p, stream);
-      case 32: return launch_grp<Tag, 32>(p, stream);
       default: break;
     }
   }

@@ -797,7 +797,8 @@ def test_attn_latent_edges(tmo, ref, dev, Hq, S, BS, dtype):
 def test_attn_many_columns(tmo, ref, dev, kv, D, Hq, S, dtype, scales):
     """The many-column kernel over its kinds and head sizes: contexts at the edges of its 32- and
     64-key tiles, missing pages, a window, a sink, a negative softmax scale, ragged counts with
-    rows of no sequence, one split and several."""
+    rows of no sequence, one split and several (an announced maximum of 12000 keys puts the whole
+    head sizes past the kernel's lower limit)."""
     lens = [70, 1, 16, 64, 65, 127, 1500]
     case = W.attn_case(dtype, 160 + D, kv=kv, B=7, Hq=Hq, Hkv=2, D=D, BS=16, NB=700, max_ctx=1500,
                        scale_dtype=scales or torch.float32)
@@ -805,11 +806,12 @@ def test_attn_many_columns(tmo, ref, dev, kv, D, Hq, S, dtype, scales):
     case.block_tables[6, 40:42] = -1
     q = W.attn_queries(dtype, 161, B=7, Hq=Hq, D=D, S=S)
     scale = D ** -0.5
-    run_attn_mq(tmo, ref, dev, case, q, scale=scale, sink=torch.linspace(-1.0, 2.0, Hq))
+    run_attn_mq(tmo, ref, dev, case, q, scale=scale, sink=torch.linspace(-1.0, 2.0, Hq), max_ctx=12000)
     run_attn_mq(tmo, ref, dev, case, q, scale=-0.5 * scale, window=50, max_ctx=0)
     counts = [S, 1, min(16, S), 0, max(0, S - 3), min(3, S), S]
     q3, cu = W.attn_queries(dtype, 162, B=7, Hq=Hq, D=D, counts=counts)
-    run_attn_mq(tmo, ref, dev, case, torch.cat([q3, q3[:2]]), cu=cu, scale=scale, max_seq_q=S)
+    run_attn_mq(tmo, ref, dev, case, torch.cat([q3, q3[:2]]), cu=cu, scale=scale, max_seq_q=S,
+                max_ctx=12000)
 
 
 def test_attn_many_columns_quantised_q_and_sparse_tables(tmo, ref, dev):
@@ -822,7 +824,7 @@ def test_attn_many_columns_quantised_q_and_sparse_tables(tmo, ref, dev):
                                      for _ in range(3)]).to(torch.int32)
     q = _q_codes(torch.int8, (3, 20, 8, 128), 172)
     for form in ("token", "group"):
-        run_attn_mq(tmo, ref, dev, case, q, q_scale=_q_scale(form, (3, 20, 8), 173))
+        run_attn_mq(tmo, ref, dev, case, q, q_scale=_q_scale(form, (3, 20, 8), 173), max_ctx=12000)
 
 
 @pytest.mark.parametrize("B", [1, 2, 64, 65])
