@@ -232,7 +232,9 @@ __global__ __launch_bounds__(256, 2) void attn_chunk(AttnParams p) {
     *reinterpret_cast<u32x4*>(base + r * kPitch + ((chunk ^ (r & G::kX)) << 4)) = w;
   };
   // Convert the rows in flight and write them to LDS buffer `buf`; rows without a key are zeros,
-  // or codes (finite) with scale 0.
+  // or integer codes with scale 0.  float8 values of no key are cleared too: whatever row 0 or a
+  // page's rest holds there may be NaN codes, and p = 0 would not remove those (K's scores of no
+  // key are replaced).
   auto stage = [&](int buf) {
 #pragma unroll
     for (int j = 0; j < G::kKL; ++j) {
@@ -272,7 +274,7 @@ __global__ __launch_bounds__(256, 2) void attn_chunk(AttnParams p) {
       const int u = tid + 256 * j, r = u / G::kVU, c = u - r * G::kVU;
       if (G::kVRows * G::kVU % 256 != 0 && u >= G::kVRows * G::kVU) continue;
       u32x4 w = vw[j];
-      if (!kQuant && !(vok >> j & 1)) w = u32x4{0u, 0u, 0u, 0u};
+      if ((!kQuant || kKind == 3) && !(vok >> j & 1)) w = u32x4{0u, 0u, 0u, 0u};
       if constexpr (!kQuant) {
         put(lds_v[buf], r, c, w);
       } else {

@@ -827,6 +827,42 @@ def test_attn_many_columns_quantised_q_and_sparse_tables(tmo, ref, dev):
         run_attn_mq(tmo, ref, dev, case, q, q_scale=_q_scale(form, (3, 20, 8), 173), max_ctx=12000)
 
 
+@pytest.mark.parametrize("kv,D,S", [("fp8_token", 80, 1), ("fp8_channel", 96, 2), ("fp8_token", 128, 16),
+                                    ("int8_token", 96, 1), ("plain", 80, 1), ("plain", 256, 16)])
+def test_attn_many_columns_ignores_what_holds_no_key(tmo, ref, dev, kv, D, S):
+    """Page 0 (of no sequence), a page whose table entry is -1 and the rest of the last pages hold
+    NaN -- values, float8 codes, per-token scales: the outputs stay the same, bit for bit."""
+    lens = [1, 15, 33, 64, 65, 700]
+    case = W.attn_case(torch.bfloat16, 190, kv=kv, B=6, Hq=8, Hkv=2, D=D, BS=16, NB=6 * 44 + 1,
+                       max_ctx=700)
+    case.block_tables = torch.arange(1, 6 * 44 + 1, dtype=torch.int32).reshape(6, 44)
+    case.context_lens = torch.tensor(lens, dtype=torch.int32)
+    case.block_tables[5, 3] = -1
+    q = W.attn_queries(torch.bfloat16, 191, B=6, Hq=8, D=D, S=S)
+    clean, _ = run_attn_mq(tmo, ref, dev, case, q, max_ctx=12000)
+
+    def unused(t, value):
+        t[0] = value
+        t[5 * 44 + 4] = value
+        for i, n in enumerate(lens):
+            t[1 + i * 44 + (n - 1) // 16, :, (n - 1) % 16 + 1:] = value
+
+    for cache in (case.k_cache, case.v_cache):
+        if kv.startswith("fp8"):
+            unused(cache.view(torch.uint8), 0x7f)
+        elif kv == "plain":
+            unused(cache, float("nan"))
+    if kv.endswith("token"):
+        unused(case.k_scale, float("nan"))
+        unused(case.v_scale, float("nan"))
+    out = tmo.single_query_cached_kv_attn(
+        q.to(dev), case.k_cache.to(dev), case.v_cache.to(dev), torch.empty_like(q, device=dev),
+        case.block_tables.to(dev), case.context_lens.to(dev),
+        None if kv == "plain" else case.k_scale.to(dev), None if kv == "plain" else case.v_scale.to(dev),
+        None, 12000, -1, -1, 0.0883883, kv_cache_quant_bit_size=-1 if kv == "plain" else 8)
+    assert torch.equal(out.cpu().double(), clean)
+
+
 @pytest.mark.parametrize("B", [1, 2, 64, 65])
 @pytest.mark.parametrize("kv,D", [("plain", 64), ("int8_channel", 128), ("int4_token", 256)])
 def test_attn_ragged_over_splits(tmo, ref, dev, kv, D, B):
