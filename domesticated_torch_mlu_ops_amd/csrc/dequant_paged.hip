@@ -439,7 +439,6 @@ __global__ __launch_bounds__(256) void dequant_page_list(DequantParams p, PageEn
   list[page_start + j] = e;
 }
 
-//
 // Rows whose 8-code chunks are no power of two (head sizes 80, 96, ...; part rows, kMode with
 // kPartRow) count as the next power of two of units: the units past a row read its last chunk
 // and write nothing.  16 contexts of 1024..8192 tokens, 8 heads x 96: 273 us on the per-element
