@@ -883,3 +883,14 @@ def test_attn_ragged_over_splits(tmo, ref, dev, kv, D, B):
     q3, cu = W.attn_queries(torch.bfloat16, 182, B=B, Hq=16, D=D,
                             counts=[(i + 1) % 4 for i in range(B)])
     run_attn_mq(tmo, ref, dev, case, q3, cu=cu, max_seq_q=3)
+
+
+@pytest.mark.parametrize("D", [64, 80])
+def test_attn_merge_batches(tmo, ref, dev, D):
+    """Sequences whose keys fill 1, 16, 17, 32, 33 and 63 splits: the edges of the batches of 16
+    in which their results are merged."""
+    case = W.attn_case(torch.bfloat16, 200 + D, kv="plain", B=6, Hq=2, Hkv=1, D=D, BS=16,
+                       NB=6 * 1008, max_ctx=63 * 256)
+    case.context_lens = torch.tensor([256, 4096, 4097, 8192, 8193, 63 * 256], dtype=torch.int32)
+    q = W.attn_queries(torch.bfloat16, 201, B=6, Hq=2, D=D, S=1)
+    run_attn_mq(tmo, ref, dev, case, q)
