@@ -384,7 +384,9 @@ __global__ __launch_bounds__(256, 2) void attn_chunk(AttnParams p) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) qabs = fmaxf(qabs, fabsf(x[m][e]));
     }
-    // The column's factor is positive (maxima of the unscaled scores); its sign goes into q
+    // The column's factor is positive (maxima of the unscaled scores, and masked scores stay -inf
+    // under it): its sign goes into q, and so does a factor of zero (a zero softmax scale, the
+    // zero scale of an all-zero q row), whose product with -inf would be NaN
     const float q_rs = (kQuant && qvalid[cb] && p.qs_mode) ? q_row_scale(p, qse) : 1.0f;
     float sigma = 1.0f, inv_sigma = 1.0f;
     if constexpr (kQuant) {
@@ -397,6 +399,10 @@ __global__ __launch_bounds__(256, 2) void attn_chunk(AttnParams p) {
     if (sscale[cb] < 0.0f) {
       sscale[cb] = -sscale[cb];
       sigma = -sigma;
+    }
+    if (sscale[cb] == 0.0f) {
+      sscale[cb] = 1.0f;
+      sigma = 0.0f;
     }
 #pragma unroll
     for (int m = 0; m < kQM; ++m)
@@ -502,9 +508,7 @@ __global__ __launch_bounds__(256, 2) void attn_chunk(AttnParams p) {
       for (int t = 0; t < kTT; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) tmax = fmaxf(tmax, s[cb][t][e]);
-      tmax = col_max_swap(tmax);
-      // a zero factor would make -inf a NaN
-      tmax = tmax == -__builtin_inff() ? tmax : tmax * cs;
+      tmax = col_max_swap(tmax) * cs;
       // the lazily moved maximum of attn_mfma
       const bool was_empty = mrun[cb] == -__builtin_inff();
       const bool raise = tmax > mrun[cb] + kLazy || (was_empty && tmax != -__builtin_inff());

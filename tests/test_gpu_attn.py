@@ -863,6 +863,34 @@ def test_attn_many_columns_ignores_what_holds_no_key(tmo, ref, dev, kv, D, S):
     assert torch.equal(out.cpu().double(), clean)
 
 
+@pytest.mark.parametrize("kv,D,S", [("int8_token", 96, 1), ("fp8_token", 80, 9), ("int8_token", 128, 20),
+                                    ("int8_channel", 64, 20), ("int4_token", 256, 20), ("plain", 96, 2),
+                                    ("plain", 128, 20), ("plain", 256, 20)])
+def test_attn_many_columns_zero_factor(tmo, ref, dev, kv, D, S):
+    """A query column whose scores are all zero (a zero softmax scale; an all-zero q row with the
+    scale 0 that the quantisers store for it) attends evenly to the keys it sees and to no masked
+    one: context tails, causal edges, a window and missing pages, one split and several."""
+    lens = [70, 1, 16, 64, 65, 127, 1500]
+    case = W.attn_case(torch.bfloat16, 210 + D, kv=kv, B=7, Hq=8, Hkv=2, D=D, BS=16, NB=700,
+                       max_ctx=1500)
+    case.context_lens = torch.tensor(lens, dtype=torch.int32)
+    case.block_tables[6, 40:42] = -1
+    q = W.attn_queries(torch.bfloat16, 211, B=7, Hq=8, D=D, S=S)
+    for scale in (0.0, -0.0):
+        run_attn_mq(tmo, ref, dev, case, q, scale=scale, max_ctx=12000)
+        run_attn_mq(tmo, ref, dev, case, q, scale=scale, window=50, max_ctx=12000)
+    if kv == "plain":
+        return
+    for qdt in (torch.int8, torch.float8_e4m3fn):
+        codes = _q_codes(qdt, (7, S, 8, D), 212)
+        scales = _q_scale("token", (7, S, 8), 213)
+        for i, s, h in ((0, 0, 0), (3, S - 1, 5), (6, 0, 7), (6, S // 2, 2)):
+            codes[i, s, h] = 0
+            scales[i, s, h] = 0.0
+        run_attn_mq(tmo, ref, dev, case, codes, q_scale=scales, max_ctx=12000)
+        run_attn_mq(tmo, ref, dev, case, codes, q_scale=scales, window=50, max_ctx=12000)
+
+
 @pytest.mark.parametrize("B", [1, 2, 64, 65])
 @pytest.mark.parametrize("kv,D", [("plain", 64), ("int8_channel", 128), ("int4_token", 256)])
 def test_attn_ragged_over_splits(tmo, ref, dev, kv, D, B):
