@@ -281,6 +281,16 @@ __device__ __forceinline__ float col_sum(float v) {
   return v + __shfl_xor(v, 32, kWave);
 }
 
+// The 16-bit values of dword w that are no number (all exponent bits set) cleared; nonzero where
+// there was one.
+template <bool kF16>
+__device__ __forceinline__ uint32_t clear_non_numbers(uint32_t& w) {
+  // the magnitude's carry into the sign's place
+  const uint32_t hit = ((w & 0x7fff7fffu) + (kF16 ? 0x04000400u : 0x00800080u)) & 0x80008000u;
+  w &= ~((hit >> 15) * 0xffffu);
+  return hit;
+}
+
 // ------------------------------------------------------------------------------ MFMA kernel
 
 template <bool kF16>

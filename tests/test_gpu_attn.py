@@ -774,6 +774,45 @@ def test_attn_latent_edges(tmo, ref, dev, Hq, S, BS, dtype):
     assert torch.equal(out.cpu().double(), clean)
 
 
+def _attn_call(tmo, dev, case, q, Dv, scale, window, max_ctx, int4=False):
+    """The operator alone: the output on the host."""
+    on = lambda t: None if t is None else t.to(dev)  # noqa: E731
+    bits = 4 if int4 else 8 if case.k_cache.element_size() == 1 else -1
+    return tmo.single_query_cached_kv_attn(
+        q.to(dev), on(case.k_cache), on(case.v_cache),
+        torch.empty(q.shape[:-1] + (Dv,), dtype=q.dtype, device=dev), on(case.block_tables),
+        on(case.context_lens), on(case.k_scale), on(case.v_scale), None, max_ctx, window, -1, scale,
+        kv_cache_quant_bit_size=bits).cpu()
+
+
+def _masked_values(tmo, ref, dev, case, q, Dv, window, max_ctx, poison):
+    """Keys that a query token does not see may hold anything: with the rows before every token's
+    window and then the last key (which only the last token sees) replaced by `poison(i, rows)`,
+    the tokens that see none of them keep their outputs bit for bit, and the others are no
+    numbers exactly where the oracle's are none."""
+    S, lens, scale = q.shape[1], case.context_lens.tolist(), q.shape[-1] ** -0.5
+    args = (Dv, scale, window, max_ctx, case.int4)
+    vmax = _vmax(case, case.v_scale, Dv)
+    clean = _attn_call(tmo, dev, case, q, *args)
+    assert clean.isfinite().all()
+    if window >= 0:
+        for i, n in enumerate(lens):
+            poison(i, range(max(0, n - S - window)))
+        assert torch.equal(_attn_call(tmo, dev, case, q, *args), clean)
+    for i, n in enumerate(lens):
+        poison(i, [n - 1])
+    got = _attn_call(tmo, dev, case, q, *args)
+    assert torch.equal(got[:, :-1], clean[:, :-1])
+    want, _ = ref.cached_kv_attn(q, case.k_cache, case.v_cache, case.block_tables, case.context_lens,
+                                 scale, case.k_scale, case.v_scale, None, window, head_size_v=Dv,
+                                 int4=case.int4)
+    assert not want[:, -1].isfinite().all()
+    assert torch.equal(got.isfinite(), want.isfinite())
+    held = want.isfinite()
+    err = (got.double() - want).abs()[held]
+    assert (err <= RTOL[q.dtype] * want.abs()[held] + ATOL[q.dtype] * vmax).all()
+
+
 # ---------------------------------------------------------------------------- many query columns
 
 @pytest.mark.parametrize("kv,D,Hq,S,dtype,scales", [
@@ -889,6 +928,33 @@ def test_attn_many_columns_zero_factor(tmo, ref, dev, kv, D, S):
             scales[i, s, h] = 0.0
         run_attn_mq(tmo, ref, dev, case, codes, q_scale=scales, max_ctx=12000)
         run_attn_mq(tmo, ref, dev, case, codes, q_scale=scales, window=50, max_ctx=12000)
+
+
+@pytest.mark.parametrize("kv,D,S,dtype", [
+    ("plain", 96, 5, torch.bfloat16), ("plain", 80, 1, torch.float16), ("fp8_token", 80, 9, torch.bfloat16),
+    ("int8_token", 96, 1, torch.bfloat16), ("int4_token", 96, 4, torch.bfloat16),
+    ("plain", 128, 40, torch.bfloat16), ("plain", 64, 20, torch.float16), ("plain", 256, 20, torch.float16),
+    ("fp8_channel", 256, 20, torch.bfloat16), ("int8_token", 64, 40, torch.float16),
+    ("int4_token", 256, 20, torch.bfloat16)])
+@pytest.mark.parametrize("window", [-1, 37])
+def test_attn_many_columns_masked_values(tmo, ref, dev, kv, D, S, dtype, window):
+    """Values outside a token's window, or after it in its chunk, hold NaN and infinities: 16-bit
+    values, float8 codes, per-token scales."""
+    case = W.attn_case(dtype, 220 + D, kv=kv, B=3, Hq=8, Hkv=2, D=D, BS=16, NB=3 * 44, max_ctx=700)
+    case.context_lens = torch.tensor([70, 203, 700], dtype=torch.int32)
+
+    def poison(i, rows):
+        for r in rows:
+            page, value = int(case.block_tables[i, r // 16]), (float("inf"), float("-inf"), float("nan"))[i]
+            if kv == "plain":
+                case.v_cache[page, 1, r % 16, 5 + 20 * i] = value
+            elif kv == "fp8_channel":
+                case.v_cache.view(torch.uint8)[page, 1, r % 16, 5 + 20 * i] = 0x7f
+            else:
+                case.v_scale[page, 1, r % 16] = value
+
+    q = W.attn_queries(dtype, 221, B=3, Hq=8, D=D, S=S)
+    _masked_values(tmo, ref, dev, case, q, D, window, 12000, poison)
 
 
 @pytest.mark.parametrize("B", [1, 2, 64, 65])
