@@ -243,6 +243,12 @@ __global__ __launch_bounds__(256 * kCB, 2) void attn_latent(AttnParams p) {
         }
     };
     read_v(0);
+    // the largest magnitude of the scores, NaN where one is: two scores per v_maximum3_f32
+    float odd = 0.0f;
+#pragma unroll
+    for (int t = 0; t < kST; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) odd = __builtin_elementwise_maximum(odd, __builtin_fabsf(s[t][e]));
     float tmax = -__builtin_inff();
 #pragma unroll
     for (int t = 0; t < kST; ++t) {
@@ -309,9 +315,31 @@ __global__ __launch_bounds__(256 * kCB, 2) void attn_latent(AttnParams p) {
       }
     }
     lpart = lpart * corr + psum;
-    if (__ballot(corr != 1.0f && !was_empty)) {
+    if (__ballot((corr != 1.0f && !was_empty) || !(odd < __builtin_inff()))) {
 #pragma unroll
       for (int b = 0; b < kLatVB; ++b) acc[b] *= corr;
+      // A row with a channel that is no number has such a score in every column.  Where a column
+      // gives it no weight (a masked key, a score of -inf), p = 0 would not remove its values: they
+      // become zeros, which change nothing for the columns whose p is NaN.  The wavefront clears
+      // its own quarter of the tile (the swizzle stays inside it; another column block's
+      // wavefront writes the same zeros) and reads it again.
+      if (__ballot(!(odd < __builtin_inff()))) {
+        int first = lane;
+        asm volatile("" : "+v"(first));  // addresses are made here, not kept over the loop
+#pragma unroll 1
+        for (int u = first; u < kT * 16; u += kWave) {
+          u32x4* at = reinterpret_cast<u32x4*>(lds[buf] + (u >> 4) * kLatRow + (chq * 16 + (u & 15)) * 16);
+          u32x4 w = *at;
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            uint32_t x = w[k];
+            clear_non_numbers<kF16>(x);
+            w[k] = x;
+          }
+          *at = w;
+        }
+        read_v(0);
+      }
     }
     auto pv = [&](int b0) {
 #pragma unroll

@@ -813,6 +813,28 @@ def _masked_values(tmo, ref, dev, case, q, Dv, window, max_ctx, poison):
     assert (err <= RTOL[q.dtype] * want.abs()[held] + ATOL[q.dtype] * vmax).all()
 
 
+@pytest.mark.parametrize("Hq,S,dtype", [(16, 1, torch.bfloat16), (16, 3, torch.float16),
+                                        (64, 2, torch.bfloat16)])
+@pytest.mark.parametrize("window", [-1, 37])
+def test_attn_latent_masked_values(tmo, ref, dev, Hq, S, dtype, window):
+    """Latent rows outside a token's window, or after it in its chunk, hold NaN and infinities; a
+    key with an infinite channel has no weight where that makes its score -inf."""
+    case = W.attn_case(dtype, 154, kv="plain", B=3, Hq=Hq, Hkv=1, D=576, BS=16, NB=3 * 44, max_ctx=700)
+    case.context_lens = torch.tensor([70, 203, 700], dtype=torch.int32)
+    one = W.AttnCase(case.q, case.k_cache, None, None, None, case.block_tables, case.context_lens)
+
+    def poison(i, rows):
+        for r in rows:
+            at = (int(case.block_tables[i, r // 16]), 0, r % 16)
+            if len(rows) == 1:
+                one.k_cache[at][5 + 100 * i] = float("inf")
+            else:
+                one.k_cache[at] = float("nan")
+
+    q = W.attn_queries(dtype, 155, B=3, Hq=Hq, D=576, S=S)
+    _masked_values(tmo, ref, dev, one, q, 512, window, 700, poison)
+
+
 # ---------------------------------------------------------------------------- many query columns
 
 @pytest.mark.parametrize("kv,D,Hq,S,dtype,scales", [
