@@ -30,8 +30,8 @@ HIP_LIB = LIB_DIR / "libtmo_hip.so"
 TORCH_EXT = LIB_DIR / "_tmo_torch.so"
 
 HIP_SOURCES = ["quant_paged.hip", "reshape_paged.hip", "dequant_paged.hip", "fused_rope.hip",
-               "linear_cache.hip", "decode_attn.hip", "attn_latent.hip",
-               "attn_chunk.hip",
+               "linear_cache.hip", "decode_attn.hip", "attn_mfma_int8.hip", "attn_mfma_fp8.hip",
+               "attn_mfma_int4.hip", "attn_mfma_plain.hip", "attn_latent.hip", "attn_chunk.hip",
                "scaled_quantize.hip", "abi_info.hip"]
 
 ROCM = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))

@@ -1,6 +1,6 @@
-// Shared by the attention kernels (decode_attn.hip, attn_latent.hip,
-// attn_chunk.hip): the launch parameters, the
-// sequence and key-range rules, the softmax's last step, and the MFMA operand conversions.
+// Shared by the attention kernels (decode_attn.hip, attn_mfma.h, attn_latent.hip, attn_chunk.hip):
+// the launch parameters, the sequence and key-range rules, the softmax's last step, and the MFMA
+// operand conversions.
 #pragma once
 
 #include "attn_rules.h"
@@ -398,6 +398,12 @@ __device__ __forceinline__ void store_out4(const AttnParams& p, int64_t e, f32x4
   for (int k = 0; k < 4; ++k) store_out(p, e + k, v[k]);
 }
 
+// The MFMA kernel over each kind of cache (attn_mfma_*.hip): p.splits partials per column when > 1;
+// qlo: q needs a lo operand.
+int launch_attn_int8(const AttnParams& p, bool qlo, hipStream_t st);
+int launch_attn_fp8(const AttnParams& p, bool qlo, hipStream_t st);
+int launch_attn_int4(const AttnParams& p, bool qlo, hipStream_t st);
+int launch_attn_plain(const AttnParams& p, hipStream_t st);
 // The latent-cache kernel (attn_latent.hip): p.splits partials per column when > 1, as
 // attn_mfma leaves them.
 int launch_attn_latent(const AttnParams& p, hipStream_t st);
