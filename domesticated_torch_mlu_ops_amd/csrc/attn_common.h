@@ -208,9 +208,12 @@ struct Work {
 // and numbers them first, so the live ones are spread evenly.  Ragged contexts of 512 keys to the
 // maximum, 3-D -> packed: 4 sequences to 8192 keys (32 / 8 heads x 128, int8) 31.8 -> 26.9 us,
 // 32 to 4096 (bf16) 81.0 -> 77.3 us, 32 to 8192 on latent rows with 64 heads 108.6 -> 93.7 us;
-// 64 sequences, whose workgroups run in many rounds, 467.3 -> 465.4 us.
+// 64 sequences, whose workgroups run in many rounds, 467.3 -> 465.4 us.  kPacked is p.packed: a
+// choice inside attn_mfma cost the calls of one split, a few hundred keys long, 0.2 to 0.4 us (4
+// sequences of up to 250 int8 keys, head size 128: 13.2 us, 12.9 with an instance of each).
+template <bool kPacked>
 __device__ __forceinline__ bool work_of(const AttnParams& p, int ncb, Work& w) {
-  if (!p.packed) {
+  if constexpr (!kPacked) {
     w.i = blockIdx.z;
     w.hk = blockIdx.y;
     w.cb = (int)(blockIdx.x / (unsigned)p.splits);

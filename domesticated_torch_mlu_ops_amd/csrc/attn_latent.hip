@@ -86,7 +86,11 @@ __global__ __launch_bounds__(256 * kCB, 2) void attn_latent(AttnParams p) {
   const int chq = wave & 3;           // quarter of the value channels, and:
   const int st_tile = chq % kST, st_half = chq / kST;  // score tile, part of its channels
   Work wk;
-  if (!work_of(p, (p.ncb + kCB - 1) / kCB, wk)) return;
+  if (p.packed) {
+    if (!work_of<true>(p, (p.ncb + kCB - 1) / kCB, wk)) return;
+  } else {
+    work_of<false>(p, (p.ncb + kCB - 1) / kCB, wk);
+  }
   const int64_t i = wk.i;
   const int hk = wk.hk, split = wk.split;
   const int cbg = wk.cb;  // group of kCB column blocks

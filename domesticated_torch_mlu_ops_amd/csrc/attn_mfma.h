@@ -42,7 +42,8 @@ namespace {
 // channels, V pairing the rows of a page; f16 QK through int4_f16, bf16 PV of the exact
 // codes).  kQLo: q needs a lo operand.  kSB: the scale tensors are bf16 (else fp32).  kMask:
 // a mask is given (its terms are added in the tiles that reach the last mask_len keys; the
-// instances without one carry none of that code and its registers).
+// instances without one carry none of that code and its registers).  kPacked: the workgroups are
+// numbered live ones first (work_of).
 // Workgroups per CU the register allocation must allow: three (168 registers per lane) for
 // the quantised-cache kernels up to head_size 128, fewer where that would spill.
 constexpr bool attn_quant(int kind) { return kind == 0 || kind == 3 || kind == 4; }
@@ -54,7 +55,7 @@ constexpr int attn_min_blocks(int d, int kind) {
 #define TMO_ATTN_DEPTH 2
 #endif
 
-template <int kD, int kKind, bool kQLo, bool kSB, bool kMask>
+template <int kD, int kKind, bool kQLo, bool kSB, bool kMask, bool kPacked>
 __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(AttnParams p) {
   constexpr bool kQuant = attn_quant(kKind);  // codes with per-token / per-channel scales
   // tiles in flight per wavefront: three register sets where they fit the register budget of
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
   const int grp = lane >> 4;        // lane group c
   auto k_channel = [&](int c) -> int { return (c / kKV * 4 + grp) * kKV + c % kKV; };
   Work wk;
-  if (!work_of(p, p.ncb, wk)) return;
+  if (!work_of<kPacked>(p, p.ncb, wk)) return;
   const int64_t i = wk.i;
   const int hk = wk.hk, split = wk.split;
   const int cb = wk.cb;  // column block
@@ -670,16 +671,22 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
   if (direct && grp == 0 && p.lse) p.lse[i * p.lse_sb + qrow * p.lse_ss + (int64_t)hq * p.lse_sh] = lse_v;
 }
 
+template <int kD, int kKind, bool kQLo, bool kSB>
+int launch_mfma_q(const AttnParams& p, hipStream_t st) {
+  const dim3 grid = attn_grid(p, p.ncb), block(256);
+  if (p.packed)
+    return p.mask ? launch_kernel(attn_mfma<kD, kKind, kQLo, kSB, true, true>, grid, block, st, p)
+                  : launch_kernel(attn_mfma<kD, kKind, kQLo, kSB, false, true>, grid, block, st, p);
+  return p.mask ? launch_kernel(attn_mfma<kD, kKind, kQLo, kSB, true, false>, grid, block, st, p)
+                : launch_kernel(attn_mfma<kD, kKind, kQLo, kSB, false, false>, grid, block, st, p);
+}
+
 template <int kD, int kKind, bool kSB>
 int launch_mfma_d(const AttnParams& p, bool qlo, hipStream_t st) {
-  const dim3 grid = attn_grid(p, p.ncb), block(256);
   if constexpr (attn_quant(kKind)) {  // q of 16-bit caches is their own type: no lo operand
-    if (qlo)
-      return p.mask ? launch_kernel(attn_mfma<kD, kKind, true, kSB, true>, grid, block, st, p)
-                    : launch_kernel(attn_mfma<kD, kKind, true, kSB, false>, grid, block, st, p);
+    if (qlo) return launch_mfma_q<kD, kKind, true, kSB>(p, st);
   }
-  return p.mask ? launch_kernel(attn_mfma<kD, kKind, false, kSB, true>, grid, block, st, p)
-                : launch_kernel(attn_mfma<kD, kKind, false, kSB, false>, grid, block, st, p);
+  return launch_mfma_q<kD, kKind, false, kSB>(p, st);
 }
 
 template <int kKind, bool kSB>
