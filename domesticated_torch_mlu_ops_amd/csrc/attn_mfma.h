@@ -8,9 +8,9 @@
 // of 16.  A workgroup of four wavefronts owns one (sequence, KV head, split, column block) and its
 // wavefronts take every fourth 16-token tile.  Per tile:
 //   * S^T = K Q^T with v_mfma_f32_16x16x16 (tokens are the rows, the block's query columns the
-//     columns, zero-padded to 16): lane (t = l % 16, c = l / 16) holds every fourth 16-byte
-//     vector of token t's row from vector c on, and MFMA m takes channels 4m .. + 3 of every
-//     lane group's own (a permutation of the reduction order).
+//     columns, zero-padded to 16): lane (t = l % 16, c = l / 16) holds a quarter of token t's
+//     row (one run of channels, or every fourth 16-byte vector: k_channel), and MFMA m takes
+//     channels 4m .. + 3 of every lane group's own (a permutation of the reduction order).
 //     Int8 codes enter as exact f16 values 1152 + code (two byte permutes per four codes) against
 //     a power-of-two scaled f16 q, and 1152 * sum(q) is subtracted from the fp32 result; the
 //     per-token scale and softmax_scale * log2(e) then multiply it.  Int4 codes enter as
@@ -65,17 +65,20 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
   using M = Mfma<kF16>;
   using V4 = typename M::V4;
   constexpr int kDC = kD / 4;       // channels per lane group in the K layout
-  // K channels per vector load of a lane.  The lane groups' vectors alternate along the row, so
-  // one load of the wavefront covers 64 contiguous bytes of each token: channel c of a lane's kDC
-  // is channel k_channel(c) of the row.  With one contiguous run of the row per lane, the loads of
-  // rows longer than 64 bytes strode over it, a quarter (bf16, 128 channels) of each 64-byte line
-  // at a time: 8 sequences of 128..4096 keys, 32 / 8 heads x 128 bf16: 39.5 -> 34.0 us, 32
-  // sequences of 512..4096 keys: 95 -> 77 us (int8 rows of 128 bytes: level).
-  constexpr int kKV = (kKind == 1 || kKind == 2) ? 8 : kKind == 4 ? (kDC < 32 ? kDC : 32) : 16;
   constexpr int kDV = kD / 16;      // channels per lane in the V layout
   constexpr int kQK = kD / 16;      // QK MFMAs per tile
   constexpr int kEs = kQuant ? 1 : 2;  // cache element bytes
   constexpr bool kInt4 = kKind == 4;
+  // Channel c of a lane's kDC is channel k_channel(c) of the row: runs of kKV channels, the lane
+  // groups' runs in turn.  Rows of more than 128 bytes take runs of one 16-byte vector, so one
+  // load of the wavefront covers 64 contiguous bytes of each token; with one run per lane it strode
+  // over them, a quarter (bf16, 128 channels) of each 64-byte line at a time: 8 sequences of
+  // 128..4096 keys, 32 / 8 heads x 128 bf16: 39.5 -> 34.0 us, 32 sequences of 512..4096 keys: 95 ->
+  // 77 us.  Shorter rows take one run per lane: int8 and float8 rows of 128 bytes measured 0.2 to
+  // 0.5 us longer in alternating vectors (4 sequences of up to 250 keys: 12.9 and 12.5 us against
+  // 12.7 and 12.0).
+  constexpr bool kAlt = !kInt4 && kD * kEs > 128;  // (int4 rows: 128 bytes at most)
+  constexpr int kKV = kAlt ? 16 / kEs : kDC;
 
   const int lane = threadIdx.x & (kWave - 1);
   // wave-uniform (readfirstlane): the tile indices, page numbers and page offsets derived from it
@@ -101,7 +104,7 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
   const bool qvalid = c < p.ncols && token_valid(p, sq, tok);
   const int64_t qrow = sq.row0 + tok;
 
-  // ---- Q operand (B of S^T = K Q^T): column `col`, channels grp * kDC + 4m .. + 3.  The QK
+  // ---- Q operand (B of S^T = K Q^T): column `col`, channels k_channel(4m .. 4m + 3).  The QK
   // product runs on f16 operands: int8 codes as 1152 + code (codes_f16), q scaled by a power
   // of two sigma that puts the column's largest |q| in [2^14, 2^15) (an f16 holds every bf16
   // and f16 value of that column exactly down to 2^-29 of the largest), with a second (lo)
@@ -284,9 +287,9 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
   constexpr int kVRow = kInt4 ? kD : kD * kEs;
   constexpr int kVRows = kInt4 ? 2 : 4;                     // V rows per lane: tokens 4 grp .. + 3
   const int64_t page_bytes = (int64_t)p.BS * kKRow;         // one head's page
-  // per-lane offsets inside a 16-row piece of a page: K token `col`, channels grp * kDC ..;
-  // V tokens 4 grp .. + 3, channels col * kDV ..
-  constexpr int kKStep = kInt4 ? kKV / 2 : kKV * kEs;       // bytes of one vector
+  // per-lane offsets inside a 16-row piece of a page: K token `col`, the lane group's first run of
+  // channels; V tokens 4 grp .. + 3, channels col * kDV ..
+  constexpr int kKStep = kInt4 ? kKV / 2 : kKV * kEs;       // bytes of one run
   const int32_t k_lane = col * kKRow + grp * kKStep;
   const int32_t v_lane = kVRows * grp * kVRow + col * kDV * (kInt4 ? 1 : kEs);
   constexpr int kKW = kInt4 ? kDC / 8 : kDC * kEs / 4;      // dwords per lane
@@ -314,7 +317,7 @@ __global__ __launch_bounds__(256, (attn_min_blocks(kD, kKind))) void attn_mfma(A
     if constexpr (kKW >= 4) {
 #pragma unroll
       for (int u = 0; u < kKW / 4; ++u) {
-        const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(krow) + 4 * u);
+        const u32x4 w = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(krow) + (kAlt ? 4 * u : u));
 #pragma unroll
         for (int e = 0; e < 4; ++e) r.kw[4 * u + e] = w[e];
       }
