@@ -1010,3 +1010,15 @@ def test_attn_merge_batches(tmo, ref, dev, D):
     case.context_lens = torch.tensor([256, 4096, 4097, 8192, 8193, 63 * 256], dtype=torch.int32)
     q = W.attn_queries(torch.bfloat16, 201, B=6, Hq=2, D=D, S=1)
     run_attn_mq(tmo, ref, dev, case, q)
+
+
+@pytest.mark.parametrize("D", [64, 80, 128, 256])
+def test_attn_merge_whole_rows(tmo, ref, dev, D):
+    """4096 output rows, each merged by one wavefront over all its channels: announced maxima of
+    3, 7 and more splits (batches of 4, 8 and 16), short, empty and one-key contexts."""
+    case = W.attn_case(torch.bfloat16, 230 + D, kv="int8_token", B=4, Hq=32, Hkv=1, D=D, BS=16,
+                       NB=4 * 38, max_ctx=600)
+    case.context_lens = torch.tensor([600, 257, 0, 40], dtype=torch.int32)
+    q = W.attn_queries(torch.bfloat16, 231, B=4, Hq=32, D=D, S=32)
+    for max_ctx in (600, 1700, 16128):
+        run_attn_mq(tmo, ref, dev, case, q, scale=D ** -0.5, max_ctx=max_ctx)
