@@ -238,7 +238,11 @@ __device__ __forceinline__ bool work_of(const AttnParams& p, int ncb, Work& w) {
   const uint32_t lv = (uint32_t)__builtin_amdgcn_readlane((int)live, s);
   const uint32_t unit = __builtin_amdgcn_readfirstlane(rem / lv);
   w.i = s;
-  w.split = (int)(rem - unit * lv);
+  // Consecutive workgroups go round the 8 XCDs.  Where the live splits divide that round, the last
+  // and shorter ones would all come to the same XCDs: every second four units count backwards (64
+  // sequences of up to 1000 int8 keys, 4 tokens: 43.5 -> 40.3 us).
+  const uint32_t nth = rem - unit * lv;
+  w.split = (int)(unit & 4 ? lv - 1 - nth : nth);
   w.hk = (int)(__builtin_amdgcn_readfirstlane(unit / (uint32_t)ncb));
   w.cb = (int)(unit - (uint32_t)w.hk * (uint32_t)ncb);
   w.sq.L = __builtin_amdgcn_readlane((int)own.L, s);
