@@ -550,25 +550,16 @@ extern "C" int tmo_hip_cached_kv_attn(
                       head_size_v == 512 && k_cache_dim == 576 && block_size % 8 == 0 && p.q_vec &&
                       al(k_cache, 16) &&
                       (block_table_heads != num_q_heads || num_q_heads == num_kv_heads);
-  // Four column blocks and more (49 columns) with more than five million (query column, key) pairs over the
-  // KV heads (attn_large) take attn_chunk, which unpacks a key once for 64 or 128 columns.  8 KV heads x 128, int8 pages, contexts of 512..8192, attn_mfma against it: 32
-  // columns of 4 / 32 sequences 53 / 160 against 54 / 183 us, 64 columns 72 / 267 against 55 /
-  // 193, 128 columns (32 sequences) 492 against 212, 2048 columns of 8 sequences 1210 against 437.
-  // Its workgroups walk their keys in one chain where attn_mfma's four wavefronts share them, so
-  // short or few sequences stay there: 1 / 8 sequences of 512 keys, 64 columns, 8 KV heads, 18.8 /
-  // 19.4 against 26.9 / 27.8 us; 8 of 1024 (4.2 million pairs) 29.8 against 34.8 us, of 2048
-  // 56.3 against 39.3; 288 columns, 2 KV heads, 8 of 1024 (4.7) 30.8 against 35.5, of 2048 51.0
-  // against 42.0 us.
-  // Head sizes 80 and 96 take it with any number of columns (attn_mfma has no instance of them),
-  // but for fp32 outputs, where the VALU kernel's fp32 probabilities show: 16 sequences of
+  // Many query columns (attn_many_columns) and head sizes 80 and 96 take attn_chunk, but for fp32
+  // outputs of the latter, where the VALU kernel's fp32 probabilities show: 16 sequences of
   // 512..8192 int8 keys, 32 heads x 96, one token each, 12486 us there, 104 here.
   // It indexes cache rows and scales with 32 bits and has no mask or ALiBi terms.
-  const bool large = attn_large(p.ncols, num_kv_heads, batch, max_context_len,
-                                max_blocks * block_size);
   auto scale_span = [&](int64_t sb, int64_t sh) {
     return num_blocks * sb + num_kv_heads * sh + block_size;
   };
-  const bool chunk = mfma && (whole ? ncb >= 4 && large : out_dtype != TMO_DTYPE_F32) && !mask && !alibi_slopes &&
+  const bool chunk = mfma && (whole || out_dtype != TMO_DTYPE_F32) && !mask && !alibi_slopes &&
+                     attn_many_columns(quant, int4, head_size, p.ncols, num_kv_heads, batch,
+                                       max_context_len, max_blocks * block_size, splits) &&
                      num_kv_heads * splits * ((p.ncols + 63) / 64) <= 0x7fffffffLL &&
                      num_blocks * num_kv_heads * block_size <= 0x7fffffffLL &&
                      (!quant || scale_mode != 1 ||

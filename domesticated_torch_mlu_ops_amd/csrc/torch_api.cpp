@@ -1378,15 +1378,14 @@ void single_query_cached_kv_attn(const torch::Tensor& q_ori, const torch::Tensor
   // 109, 124, 144 us; one sequence of 8192, 16 heads, 9, 25, 47: 49, 26, 21 us.
   const bool latent = !v_cache.has_value() && !int8 && !same_as_q && D == 576 && Dv == 512;
   const int64_t cols = seq_q * (Hq / Hkv);
-  // Many query columns (attn_large), or head sizes 80 and 96 (attn_chunk: 128 columns a
-  // workgroup, 64 of head size 256 or of a q folded with scales; 512 workgroups fit the chip):
-  // about two rounds of workgroups.  512 columns of 4
+  // Many query columns (attn_chunk: 128 columns a workgroup, 64 of head size 256 or of a q folded
+  // with scales; 512 workgroups fit the chip): about two rounds of workgroups.  512 columns of 4
   // sequences x 8 KV heads, contexts to 8192, splits 1, 3, 5, 9: 282, 174, 122, 166 us; 128
   // columns, splits 3, 5, 9, 17: 112, 76, 63, 50 us; 2048 columns of 8 sequences, 1, 3, 5: 437,
   // 560, 587 us.
-  const bool large = tmo::attn_large(cols, Hkv, B, max_ctx, block_tables.size(-1) * BS);
   const bool many = !latent && !mask_p && !alibi && D == Dv && qdt != TMO_DTYPE_F32 &&
-                    (D == 80 || D == 96 || (large && cols > 48 && (D == 64 || D == 128 || D == 256)));
+                    tmo::attn_many_columns(int8 || same_as_q, int4, D, cols, Hkv, B, max_ctx,
+                                           block_tables.size(-1) * BS, max_ctx > 0 ? 2 : 1);
   const int64_t wide = D == 256 || smode == 2 || qs_mode == 3 ? 64 : 128;
   const int64_t groups = latent ? (cols <= 16 ? 1 : (cols + 31) / 32)
                          : many ? (cols + wide - 1) / wide : (cols + 15) / 16;

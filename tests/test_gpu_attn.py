@@ -837,13 +837,28 @@ def test_attn_latent_masked_values(tmo, ref, dev, Hq, S, dtype, window):
 
 # ---------------------------------------------------------------------------- many query columns
 
+def _many_columns(case, Hq, S, max_ctx):
+    """attn_many_columns of csrc/attn_rules.h: the call goes to the many-column kernel."""
+    Hkv, D = case.k_cache.shape[1], case.q.shape[-1]
+    if D in (80, 96):
+        return not (case.int4 and D == 80)
+    cols, seqs = S * Hq // Hkv, Hkv * case.context_lens.numel()
+    keys = max_ctx or case.block_tables.shape[-1] * 16
+    blocks = (cols + 15) // 16
+    if blocks < 4 or cols * seqs * keys <= 5e6:
+        return False
+    if D == 64 and case.k_scale is not None:
+        return blocks >= 7 and blocks * seqs >= 2048
+    return max_ctx > 256 or blocks * seqs >= 1024
+
+
 @pytest.mark.parametrize("kv,D,Hq,S,dtype,scales", [
     ("int8_token", 128, 8, 13, torch.bfloat16, torch.float32),     # 52 columns: one wavefront short
     ("int8_token", 128, 8, 33, torch.float16, torch.bfloat16),     # 132: a second workgroup
     ("int8_channel", 128, 8, 17, torch.bfloat16, torch.float32),   # q folded: lo operand
-    ("int8_token", 64, 16, 40, torch.bfloat16, torch.float32),
     ("fp8_token", 256, 8, 16, torch.bfloat16, torch.float32),
-    ("fp8_channel", 64, 8, 16, torch.float16, torch.bfloat16),
+    ("fp8_channel", 128, 8, 16, torch.float16, torch.bfloat16),
+    ("plain", 64, 16, 40, torch.bfloat16, None),
     ("int4_token", 128, 8, 20, torch.bfloat16, torch.float32),
     ("int4_channel", 256, 8, 13, torch.float16, torch.float32),
     ("int8_token", 80, 8, 2, torch.float16, torch.float32),        # 8 columns, padded channels
@@ -865,6 +880,7 @@ def test_attn_many_columns(tmo, ref, dev, kv, D, Hq, S, dtype, scales):
                        scale_dtype=scales or torch.float32)
     case.context_lens = torch.tensor(lens, dtype=torch.int32)
     case.block_tables[6, 40:42] = -1
+    assert _many_columns(case, Hq, S, 12000)
     q = W.attn_queries(dtype, 161, B=7, Hq=Hq, D=D, S=S)
     scale = D ** -0.5
     run_attn_mq(tmo, ref, dev, case, q, scale=scale, sink=torch.linspace(-1.0, 2.0, Hq), max_ctx=12000)
@@ -873,6 +889,34 @@ def test_attn_many_columns(tmo, ref, dev, kv, D, Hq, S, dtype, scales):
     q3, cu = W.attn_queries(dtype, 162, B=7, Hq=Hq, D=D, counts=counts)
     run_attn_mq(tmo, ref, dev, case, torch.cat([q3, q3[:2]]), cu=cu, scale=scale, max_seq_q=S,
                 max_ctx=12000)
+
+
+@pytest.mark.parametrize("kv,D", [("int8_token", 128), ("fp8_channel", 128), ("int4_token", 256),
+                                  ("plain", 64), ("int8_channel", 96)])
+def test_attn_many_columns_one_split(tmo, ref, dev, kv, D):
+    """The many-column kernel with an unknown maximum, so one split: contexts at the edges of its
+    tiles, a window, a negative scale."""
+    case = W.attn_case(torch.bfloat16, 175 + D, kv=kv, B=7, Hq=8, Hkv=2, D=D, BS=16, NB=7 * 20,
+                       max_ctx=310)
+    case.context_lens = torch.tensor([310, 1, 63, 64, 65, 129, 300], dtype=torch.int32)
+    pad = torch.full((7, 300), -1, dtype=torch.int32)  # wide tables: what an unknown maximum may be
+    case.block_tables = torch.cat([case.block_tables, pad], dim=1).contiguous()
+    q = W.attn_queries(torch.bfloat16, 176, B=7, Hq=8, D=D, S=300)
+    assert _many_columns(case, 8, 300, 0)
+    run_attn_mq(tmo, ref, dev, case, q, scale=-(D ** -0.5), window=50, max_ctx=0)
+
+
+@pytest.mark.parametrize("kv,dtype", [("int8_token", torch.float16), ("int8_channel", torch.bfloat16),
+                                      ("fp8_token", torch.bfloat16), ("int4_token", torch.bfloat16)])
+def test_attn_many_columns_codes_of_64(tmo, ref, dev, kv, dtype):
+    """The many-column kernel over codes of head size 64, which takes many sequences: short contexts
+    at the edges of its tiles, a window, a zero scale."""
+    case = W.attn_case(dtype, 178, kv=kv, B=64, Hq=8, Hkv=2, D=64, BS=16, NB=64 * 9, max_ctx=140)
+    case.context_lens = torch.tensor([(i * 13) % 140 + 1 for i in range(62)] + [0, 140], dtype=torch.int32)
+    q = W.attn_queries(dtype, 179, B=64, Hq=8, D=64, S=64)
+    assert _many_columns(case, 8, 64, 12000)
+    run_attn_mq(tmo, ref, dev, case, q, scale=0.125, max_ctx=12000)
+    run_attn_mq(tmo, ref, dev, case, q, scale=0.0, window=30, max_ctx=12000)
 
 
 def test_attn_many_columns_quantised_q_and_sparse_tables(tmo, ref, dev):
@@ -925,7 +969,7 @@ def test_attn_many_columns_ignores_what_holds_no_key(tmo, ref, dev, kv, D, S):
 
 
 @pytest.mark.parametrize("kv,D,S", [("int8_token", 96, 1), ("fp8_token", 80, 9), ("int8_token", 128, 20),
-                                    ("int8_channel", 64, 20), ("int4_token", 256, 20), ("plain", 96, 2),
+                                    ("int8_channel", 128, 20), ("int4_token", 256, 20), ("plain", 96, 2),
                                     ("plain", 128, 20), ("plain", 256, 20)])
 def test_attn_many_columns_zero_factor(tmo, ref, dev, kv, D, S):
     """A query column whose scores are all zero (a zero softmax scale; an all-zero q row with the
@@ -956,7 +1000,7 @@ def test_attn_many_columns_zero_factor(tmo, ref, dev, kv, D, S):
     ("plain", 96, 5, torch.bfloat16), ("plain", 80, 1, torch.float16), ("fp8_token", 80, 9, torch.bfloat16),
     ("int8_token", 96, 1, torch.bfloat16), ("int4_token", 96, 4, torch.bfloat16),
     ("plain", 128, 40, torch.bfloat16), ("plain", 64, 20, torch.float16), ("plain", 256, 20, torch.float16),
-    ("fp8_channel", 256, 20, torch.bfloat16), ("int8_token", 64, 40, torch.float16),
+    ("fp8_channel", 256, 20, torch.bfloat16), ("int8_token", 128, 40, torch.float16),
     ("int4_token", 256, 20, torch.bfloat16)])
 @pytest.mark.parametrize("window", [-1, 37])
 def test_attn_many_columns_masked_values(tmo, ref, dev, kv, D, S, dtype, window):
