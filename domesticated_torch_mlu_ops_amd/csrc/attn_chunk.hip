@@ -136,9 +136,10 @@ __global__ __launch_bounds__(256, kD <= 64 && !chunk_quant(kKind) ? 3 : 2) void 
   const int cbg = (int)(yr / (unsigned)p.splits);  // group of 4 kC column blocks
   const int split = (int)yr - cbg * p.splits;
   const Seq sq = seq_of(p, i);
-  const Range rg = token_range(p, sq, split);
+  const int64_t per = fitted_split(p);
+  const Range rg = token_range(p, sq, split, per);
   if (p.splits > 1 && rg.begin >= rg.end) return;  // an empty split writes no partial
-  const bool direct = live_splits(p, sq) <= 1;     // no merge: the only split writes the output
+  const bool direct = live_splits(p, sq, per) <= 1;     // no merge: the only split writes the output
 
   // the workgroup's keys: from its first token's window start to its last token's position
   constexpr int kCols = 64 * kC;

@@ -67,6 +67,7 @@ struct AttnParams {
   int32_t splits;
   int32_t packed;                // 1-D grid, live workgroups first (work_of)
   int32_t lone;                  // a sequence's only live split writes the output itself
+  int32_t few;                   // many columns: splits that leave a CU at most one workgroup, or 0
   int64_t split_tokens;          // multiple of 64 (latent caches: 32)
   float* ws;                     // [B, Hkv, splits, ncols, Dv + 2] when splits > 1
 };
@@ -174,24 +175,46 @@ struct Range {
   int64_t begin, end;
 };
 
-__device__ __forceinline__ Range token_range(const AttnParams& p, const Seq& q, int s) {
+__device__ __forceinline__ Range token_range(const AttnParams& p, const Seq& q, int s, int64_t per) {
   Range r;
   const int64_t L = q.L;
   int64_t j0 = 0;
   if (p.window >= 0 && L - q.nq - p.window > 0) j0 = L - q.nq - p.window;
-  r.begin = j0 + (int64_t)s * p.split_tokens;
-  r.end = r.begin + p.split_tokens < L ? r.begin + p.split_tokens : L;
+  r.begin = j0 + (int64_t)s * per;
+  r.end = r.begin + per < L ? r.begin + per : L;
   if (s == p.splits - 1) r.end = L;  // the last split takes any tokens past max_context_len
   if (p.splits == 1) r.begin = j0;
   return r;
 }
+__device__ __forceinline__ Range token_range(const AttnParams& p, const Seq& q, int s) {
+  return token_range(p, q, s, p.split_tokens);
+}
 
-// Splits of the sequence that hold keys: a prefix of the launch's (the others write nothing).
-__device__ __forceinline__ int live_splits(const AttnParams& p, const Seq& q) {
-  if (p.splits <= 1 || p.split_tokens <= 0) return p.splits;
-  const int64_t left = q.L - token_range(p, q, 0).begin;
-  const int64_t n = (left + p.split_tokens - 1) / p.split_tokens;
-  return left <= 0 ? 0 : (int)(n < p.splits ? n : p.splits);
+// The many-column kernel's keys per split: as many as the split counts for the longest context
+// present would give, where the announced maximum (split_tokens) gives more.
+__device__ __forceinline__ int64_t fitted_split(const AttnParams& p) {
+  if (p.few < 2) return p.split_tokens;
+  uint32_t own = 0;
+  for (int j = threadIdx.x & (kWave - 1); j < p.B; j += kWave) own = max(own, (uint32_t)max(p.lens[j], 0));
+  const uint32_t longest = wave_max_u32_sgpr(own);
+  uint32_t n = (longest + 255) / 256;
+  if (n > 1) n -= 1 - (n & 1);
+  n = max(n, min((longest + 127) / 128, (uint32_t)p.few));
+  n = min(n, (uint32_t)p.splits);
+  const uint32_t per = n <= 1 ? longest : (longest + n - 1) / n;
+  const int64_t fit = ((int64_t)per + 63) / 64 * 64;
+  return fit > 0 && fit < p.split_tokens ? fit : p.split_tokens;
+}
+
+// Splits of the sequence that hold keys, `per` each: a prefix of the launch's (the others write
+// nothing).
+__device__ __forceinline__ int live_splits(const AttnParams& p, const Seq& q, int64_t per) {
+  if (p.splits <= 1 || per <= 0) return p.splits;
+  const int64_t left = q.L - token_range(p, q, 0, per).begin;
+  if (left <= 0) return 0;
+  if (left <= per) return 1;
+  const uint32_t n = ((uint32_t)left + (uint32_t)per - 1) / (uint32_t)per;  // per < left < 2^31
+  return n < (uint32_t)p.splits ? (int)n : p.splits;
 }
 
 // A workgroup's work: split `split` of column-block group cb of KV head hk of sequence i.

@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256) void attn_combine(AttnParams p) {
   const int64_t stride = (int64_t)p.ncols * (p.Dv + 2);
   const float* base = p.ws + ((i * p.Hkv + hk) * p.splits * (int64_t)p.ncols + c) * (p.Dv + 2);
   // splits past the sequence's keys wrote nothing (the main kernel returned early)
-  const int live = live_splits(p, sq);
+  const int live = live_splits(p, sq, p.lone ? fitted_split(p) : p.split_tokens);
   if (p.lone && live == 1) return;
   // Every load is unconditional (split and channel indices clamped into this column's rows of
   // the workspace; an empty split's row is read and given weight 0), so the loads of a batch
@@ -310,8 +310,8 @@ template <int kBatch>
 int launch_combine(const AttnParams& p, hipStream_t st) {
   const int64_t rows = (int64_t)p.B * p.S * p.Hq;
   const unsigned blocks = (unsigned)((rows + 3) / 4), chunks = (unsigned)((p.Dv + kWave - 1) / kWave);
-  if (rows >= 4096 && p.splits <= kWave)
-    return launch_kernel(attn_combine<kBatch, true>, dim3(blocks), dim3(256), st, p);
+  if (rows >= (chunks > 1 ? 4096 : 16384) && p.splits <= kWave)
+    return launch_kernel(attn_combine<4, true>, dim3(blocks), dim3(256), st, p);
   return launch_kernel(attn_combine<kBatch, false>, dim3(blocks, chunks), dim3(256), st, p);
 }
 
@@ -591,6 +591,7 @@ extern "C" int tmo_hip_cached_kv_attn(
   if (chunk) {
     p.lone = 1;
     p.packed = 0;
+    p.few = p.splits > 1 ? (int32_t)(255 / (batch * num_kv_heads * ((p.ncols + 127) / 128))) : 0;
     const int rc = launch_attn_chunk(p, qlo, st);
     return rc != TMO_OK || p.splits == 1 ? rc : launch_combine(p, st);
   }

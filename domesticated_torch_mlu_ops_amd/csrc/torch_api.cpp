@@ -1392,7 +1392,8 @@ void single_query_cached_kv_attn(const torch::Tensor& q_ori, const torch::Tensor
   const int64_t pairs = B * Hkv * groups;  // workgroups of one split
   const int64_t target = latent ? 820 : many ? 1024 : 3072, least = latent ? 96 : 256;
   if (max_ctx > 0 && pairs < target) {
-    const int64_t want = latent || many ? std::max<int64_t>(1, target / pairs) : (target + pairs - 1) / pairs;
+    int64_t want = latent || many ? std::max<int64_t>(1, target / pairs) : (target + pairs - 1) / pairs;
+    if (many && want == 2) want = 1;
     const int64_t cap = (max_ctx + least - 1) / least;
     splits = std::max<int64_t>(1, std::min<int64_t>({want, cap, 63}));
     if (splits > 1 && splits % 2 == 0) splits += splits + 1 <= cap ? 1 : -1;

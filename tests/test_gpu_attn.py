@@ -919,6 +919,25 @@ def test_attn_many_columns_codes_of_64(tmo, ref, dev, kv, dtype):
     run_attn_mq(tmo, ref, dev, case, q, scale=0.0, window=30, max_ctx=12000)
 
 
+@pytest.mark.parametrize("kv,D,B,S", [("int8_token", 128, 7, 16), ("plain", 96, 7, 1), ("fp8_token", 80, 66, 1),
+                                      ("int4_token", 256, 7, 20), ("int8_channel", 128, 70, 16)])
+@pytest.mark.parametrize("longest", [63, 640, 2200])
+def test_attn_many_columns_announced(tmo, ref, dev, kv, D, B, S, longest):
+    """The keys of a split follow the longest context present where the call announces more:
+    announced maxima at, above and below it, the longest sequence past the 64th, ragged counts, a
+    window, empty sequences."""
+    case = W.attn_case(torch.bfloat16, 240 + D, kv=kv, B=B, Hq=8, Hkv=2, D=D, BS=16,
+                       NB=B * ((longest + 15) // 16), max_ctx=longest)
+    case.context_lens = torch.tensor([(i * 37) % min(longest, 300) for i in range(B)], dtype=torch.int32)
+    case.context_lens[B - 1] = longest
+    q = W.attn_queries(torch.bfloat16, 241, B=B, Hq=8, D=D, S=S)
+    for max_ctx in (longest, 2 * longest, 100000, 300):
+        run_attn_mq(tmo, ref, dev, case, q, scale=D ** -0.5, max_ctx=max_ctx)
+    run_attn_mq(tmo, ref, dev, case, q, scale=D ** -0.5, window=200, max_ctx=100000)
+    q3, cu = W.attn_queries(torch.bfloat16, 242, B=B, Hq=8, D=D, counts=[(S - i) % (S + 1) for i in range(B)])
+    run_attn_mq(tmo, ref, dev, case, q3, cu=cu, max_seq_q=S, scale=D ** -0.5, max_ctx=100000)
+
+
 def test_attn_many_columns_quantised_q_and_sparse_tables(tmo, ref, dev):
     """Quantised q (per token, and per channel group: lo operand) and per-KV-head block tables on
     the many-column kernel."""
