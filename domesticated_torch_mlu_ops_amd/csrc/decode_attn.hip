@@ -477,7 +477,7 @@ extern "C" int tmo_hip_cached_kv_attn(
   p.max_blocks = max_blocks;
   p.lens = context_lens;
   p.alibi = alibi_slopes;
-  p.window = window_left;
+  p.window = window_left < 0x7fffffffLL ? window_left : -1;  // positions are 32-bit
   p.scale_log2 = softmax_scale * kLog2e;
   p.out = out;
   p.o_sb = cu_seq_q ? 0 : out_stride_batch;

@@ -1085,3 +1085,14 @@ def test_attn_merge_whole_rows(tmo, ref, dev, D):
     q = W.attn_queries(torch.bfloat16, 231, B=4, Hq=32, D=D, S=32)
     for max_ctx in (600, 1700, 16128):
         run_attn_mq(tmo, ref, dev, case, q, scale=D ** -0.5, max_ctx=max_ctx)
+
+
+@pytest.mark.parametrize("kv,D", [("int8_token", 128), ("int8_token", 96), ("plain", 576), ("plain", 40)])
+def test_attn_wide_windows(tmo, ref, dev, kv, D):
+    """A window of 2^31 - 1 keys and more, past what 32 bits hold, is no window."""
+    case = W.attn_case(torch.bfloat16, 250 + D, kv=kv, B=4, Hq=8, Hkv=1, D=D, BS=16, NB=64, max_ctx=200)
+    if D == 576:
+        case = W.AttnCase(case.q, case.k_cache, None, None, None, case.block_tables, case.context_lens)
+    q = W.attn_queries(torch.bfloat16, 251, B=4, Hq=8, D=D, S=2)
+    for window in (2 ** 31 - 1, 2 ** 31, 2 ** 32, 2 ** 40 + 3):
+        run_attn_mq(tmo, ref, dev, case, q, scale=D ** -0.5, window=window, Dv=512 if D == 576 else None)
