@@ -404,7 +404,8 @@ __global__ __launch_bounds__(256, kD <= 64 && !chunk_quant(kKind) ? 3 : 2) void 
     float sigma = 1.0f, inv_sigma = 1.0f;
     if constexpr (kQuant) {
       qabs = col_max(qabs);
-      const int ex = qabs > 0.0f ? __builtin_amdgcn_frexp_expf(qabs) : 1;
+      // a column's largest |q| in [2^(ex-1), 2^ex); no lower than 2^-100, so that sigma stays finite
+      const int ex = qabs > 0.0f ? max(__builtin_amdgcn_frexp_expf(qabs), -100) : 1;
       sigma = __builtin_ldexpf(1.0f, 15 - ex);
       inv_sigma = __builtin_ldexpf(1.0f, ex - 15);
     }

@@ -1096,3 +1096,14 @@ def test_attn_wide_windows(tmo, ref, dev, kv, D):
     q = W.attn_queries(torch.bfloat16, 251, B=4, Hq=8, D=D, S=2)
     for window in (2 ** 31 - 1, 2 ** 31, 2 ** 32, 2 ** 40 + 3):
         run_attn_mq(tmo, ref, dev, case, q, scale=D ** -0.5, window=window, Dv=512 if D == 576 else None)
+
+
+@pytest.mark.parametrize("kv,D", [("int8_token", 128), ("int8_channel", 80), ("fp8_token", 96),
+                                  ("int4_token", 96)])
+def test_attn_tiny_queries(tmo, ref, dev, kv, D):
+    """Query rows next to zero (2^-100 to 2^-133, the bfloat16 subnormals): finite scores."""
+    case = W.attn_case(torch.bfloat16, 260 + D, kv=kv, B=3, Hq=8, Hkv=2, D=D, BS=16, NB=64, max_ctx=150)
+    q = W.attn_queries(torch.bfloat16, 261, B=3, Hq=8, D=D, S=3)
+    for i, e in enumerate((-100, -113, -116, -126, -133)):
+        q[i % 3, i // 3] = (q[i % 3, i // 3].float() * 2.0 ** e).to(torch.bfloat16)
+    run_attn_mq(tmo, ref, dev, case, q, scale=D ** -0.5)
