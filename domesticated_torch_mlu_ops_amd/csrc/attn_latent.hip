@@ -285,7 +285,9 @@ __global__ __launch_bounds__(256 * kCB, 2) void attn_latent(AttnParams p) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           const int32_t j = t0 + 16 * t + 4 * grp + e;
-          if (j >= mask_lo && j < (int32_t)sq.L) s[t][e] += mask_value(p, mask_row + (j - mask_lo)) * kLog2e;
+          // a key that the column does not see stays so, whatever its term
+          if (j >= mask_lo && j < (int32_t)sq.L && s[t][e] != -__builtin_inff())
+            s[t][e] += mask_value(p, mask_row + (j - mask_lo)) * kLog2e;
         }
     }
 #pragma unroll

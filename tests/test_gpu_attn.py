@@ -835,6 +835,22 @@ def test_attn_latent_masked_values(tmo, ref, dev, Hq, S, dtype, window):
     _masked_values(tmo, ref, dev, one, q, 512, window, 700, poison)
 
 
+@pytest.mark.parametrize("Hq", [16, 64])
+@pytest.mark.parametrize("term", [float("inf"), float("nan")])
+def test_attn_latent_mask_of_unseen_keys(tmo, ref, dev, Hq, term):
+    """Mask terms of keys that a token does not see (later in its chunk, on a missing page) are not
+    read, whatever they hold."""
+    case = W.attn_case(torch.bfloat16, 156, kv="plain", B=3, Hq=Hq, Hkv=1, D=576, BS=16, NB=3 * 20, max_ctx=300)
+    case.context_lens = torch.tensor([40, 33, 300], dtype=torch.int32)
+    case.block_tables[2, 18] = -1                                            # the last 12 keys
+    one = W.AttnCase(case.q, case.k_cache, None, None, None, case.block_tables, case.context_lens)
+    q = W.attn_queries(torch.bfloat16, 157, B=3, Hq=Hq, D=576, S=2)
+    mask = torch.randn(3, 2, 8, generator=torch.Generator().manual_seed(158))
+    mask[:, 0, 7] = term
+    mask[2] = term
+    run_attn_mq(tmo, ref, dev, one, q, mask=mask, scale=576 ** -0.5, Dv=512)
+
+
 # ---------------------------------------------------------------------------- many query columns
 
 def _many_columns(case, Hq, S, max_ctx):
