@@ -30,20 +30,7 @@
 namespace tmo {
 namespace {
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-
-template <bool kF16>
-__device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
-  if constexpr (kF16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a),
-                                                  __builtin_bit_cast(h8, b), c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a),
-                                                 __builtin_bit_cast(bf8, b), c, 0, 0, 0);
-}
 
 // Maximum over the four lane groups of a column (lanes l, l ^ 16, l ^ 32, l ^ 48), in VALU.
 __device__ __forceinline__ float col_max_swap(float v) {

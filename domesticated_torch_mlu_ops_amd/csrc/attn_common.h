@@ -342,6 +342,20 @@ struct Mfma<true> {  // f16 operands
   }
 };
 
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+
+// D = A B + C over 32 channels, bf16 or f16 operands.
+template <bool kF16>
+__device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
+  if constexpr (kF16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a),
+                                                  __builtin_bit_cast(h8, b), c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a),
+                                                 __builtin_bit_cast(bf8, b), c, 0, 0, 0);
+}
+
 // Four int8 codes (one dword) -> four f16 operands holding 1152 + code exactly: with
 // u = code + 128 (the byte with its top bit flipped), the f16 pattern 0x6400 | u is 1024 + u
 // (ulp 1 in [1024, 2048)), so two byte permutes build the four values.  The QK product then

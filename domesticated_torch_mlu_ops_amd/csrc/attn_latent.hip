@@ -40,11 +40,6 @@ constexpr int kLatVB = kLatDv / 16 / 4;   // 16-channel value blocks per wavefro
 
 __device__ __align__(16) const uint32_t kLatZeros[4] = {};
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-
 // 16 bytes per lane from global memory into LDS at byte m0 + 16 * lane of the workgroup's
 // allocation.  The caller waits for them (vmcnt) before the barrier that publishes them.  Not
 // the builtin: the compiler cannot tell the buffer being filled from the one being read and waits
@@ -53,20 +48,11 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 // between the write of m0 and its use by an LDS load.
 __device__ __forceinline__ void load_lds16(const char* base, uint32_t off, uint32_t dst) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-               :: "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(off), "s"(base) : "memory");
+               :: "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(off), "s"(base) : "memory", "m0");
 }
 __device__ __forceinline__ void load_lds16(const char* src, uint32_t dst) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
-               :: "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(src) : "memory");
-}
-
-template <bool kF16>
-__device__ __forceinline__ f32x4 mfma32(u32x4 a, u32x4 b, f32x4 c) {
-  if constexpr (kF16)
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8, a),
-                                                  __builtin_bit_cast(h8, b), c, 0, 0, 0);
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf8, a),
-                                                 __builtin_bit_cast(bf8, b), c, 0, 0, 0);
+               :: "s"(__builtin_amdgcn_readfirstlane((int)dst)), "v"(src) : "memory", "m0");
 }
 
 template <bool kF16, int kCB, bool kMask>
