@@ -7,11 +7,11 @@
 //
 // One or two wavefronts per output row, or one workgroup per row.  Every lane holds its
 // 16-byte vectors of the row in registers (all loads in flight at once), so the row is read
-// from HBM exactly once.  sq_dense_wg: rows without gather or groups of 256 * k vectors, one
+// from HBM exactly once.  sq_dense_wg: rows of 129 to 2048 vectors without gather or groups, one
 // row per workgroup at a time in a persistent grid, the smooth values of a thread's channels in
-// registers.  sq_dense: other dense rows, a grid-stride launch with a per-channel smooth vector
-// staged in LDS.  sq_grp: gathered / grouped rows (MoE) with per-channel smooth rows,
-// one staging of the group's smooth row in LDS per workgroup.  sq_vec: the remaining vector
+// registers.  sq_dense: dense rows of 64 or 128 vectors, a grid-stride launch with a per-channel
+// smooth vector staged in LDS.  sq_grp: gathered / grouped rows (MoE) with per-channel smooth
+// rows, one staging of the group's smooth row in LDS per workgroup.  sq_vec: the remaining vector
 // cases (other widths, 3-D rows, scalar or no smooth with gather / groups), the smooth vector
 // read from L2 beside the row.  A row's group (expert) is found with a wavefront prefix scan
 // of token_count and a ballot, with no host round trip.
@@ -539,7 +539,7 @@ int launch_dense(const SqParams& p, hipStream_t stream) {
 #define TMO_SQ_WG_ROW_PER_CU 3
 #endif
 
-// Dense rows of exactly 256 * kV 16-byte vectors, one row per workgroup at a time: thread t
+// Dense rows of 256 * kV 16-byte vectors (or fewer: kVP below), one row per workgroup at a time: thread t
 // owns vectors t + 256 * i of every row, so its smooth values are fixed and held in registers
 // (kV * 8 floats), a row is kV fully coalesced 4 KiB load instructions, and the workgroup's
 // next row is loaded while the current one is reduced, scaled and encoded.  The row maximum
@@ -788,10 +788,10 @@ int launch(const SqParams& p, hipStream_t stream) {
       default: return launch_dense_wg<Tag, 8 + kPartRow>(p, stream);
     }
   }
-  // Gathered / grouped rows with per-channel smooth rows: the LDS-staged kernel wherever the row
-  // is a whole number of 64-lane steps, up to 16.  Past those a row is split over two wavefronts
-  // below: staged, 14336 channels took 45.3 us for 2400 tokens (43.5 there) and 74 us for 4099
-  // (80.7), and 16.1 us for 300 (12.7).
+  // Gathered / grouped rows with per-channel smooth rows: the LDS-staged kernel for rows of 1 to 8,
+  // 10, 12, 14 and 16 64-lane steps.  Rows of other lengths up to 16 steps take sq_vec below, as do
+  // longer ones, split over two wavefronts: staged, 14336 channels took 45.3 us for 2400 tokens
+  // (43.5 there) and 74 us for 4099 (80.7), and 16.1 us for 300 (12.7).
   if (aligned && !dense && p.inner == 1 && p.smooth && p.channels > 1 &&
       p.smooth_len == p.channels && nvec % kWave == 0) {
     switch (nvec / kWave) {
