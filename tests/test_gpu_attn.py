@@ -113,11 +113,11 @@ def test_attn_per_tensor_scales(tmo, ref, dev):
 @pytest.mark.parametrize("scale_dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("kv", ["fp8_token", "fp8_channel", "fp8_group", "int8_token",
                                 "int8_channel"])
-@pytest.mark.parametrize("D", [64, 128, 256, 96])
+@pytest.mark.parametrize("D", [64, 128, 256, 96, 72])
 def test_attn_fp8_pages_and_bf16_scales(tmo, ref, dev, D, kv, scale_dtype):
     """float8_e4m3fn pages (_ops.py:868; kv_cache_quant_bit_size 8) and bf16 scale tensors
     (_ops.py:872), on the MFMA kernels (head sizes 64 / 128 / 256, per-token and per-channel
-    scales) and the VALU kernel (per-group scales, head size 96), against the float64 oracle
+    scales), the many-column kernel (96) and the VALU kernel (per-group scales, 72), against the float64 oracle
     at the stated tolerance."""
     if kv.endswith("group") and D % 32:
         pytest.skip("per-group scales need head_size % 32 == 0")
@@ -366,10 +366,10 @@ def test_attn_multi_token_cu_seq_q(tmo, ref, dev, max_seq_q):
 
 
 @pytest.mark.parametrize("Hq,Hkv,D,S", [(16, 1, 128, 3), (40, 2, 128, 2), (8, 8, 64, 6),
-                                        (8, 2, 96, 3), (8, 2, 256, 4)])
+                                        (8, 2, 96, 3), (8, 2, 72, 3), (8, 2, 256, 4)])
 def test_attn_multi_token_groups_and_head_sizes(tmo, ref, dev, Hq, Hkv, D, S):
     """Query columns over several blocks (16 x 3 = 48, 20 x 2 = 40), one head per group,
-    the generic kernel (head size 96) and head size 256."""
+    the many-column kernel (head size 96), the generic one (72) and head size 256."""
     case = W.attn_case(torch.bfloat16, 37 + Hq + D, kv="int8_token", B=3, Hq=Hq, Hkv=Hkv, D=D,
                        NB=48, max_ctx=120)
     q = W.attn_queries(torch.bfloat16, 38 + S, B=3, Hq=Hq, D=D, S=S)
@@ -642,13 +642,14 @@ def _q_scale(form, lead, seed, dtype=torch.float32, groups=4):
 
 @pytest.mark.parametrize("kv,D", [("int8_token", 128), ("int8_token", 96), ("int8_channel", 128),
                                   ("int8_channel", 96), ("fp8_token", 128), ("fp8_token", 96),
-                                  ("int4_token", 128)])
+                                  ("int4_token", 128), ("int8_token", 72), ("int8_channel", 72),
+                                  ("fp8_token", 72), ("int4_token", 80)])
 @pytest.mark.parametrize("form", ["tensor", "token", "group"])
 @pytest.mark.parametrize("qdt", [torch.int8, torch.float8_e4m3fn])
 def test_attn_quantised_q(tmo, ref, dev, qdt, form, kv, D):
     """int8 / float8_e4m3fn q with q_quant_scale per tensor, per token and head, or per channel
-    group (float32 and bfloat16 scales), over int8 / fp8 / int4 pages, on the MFMA (128) and
-    generic (96) kernels; 4-D q and cu_seq_q; the output in half (bfloat16 too for int8 q)."""
+    group (float32 and bfloat16 scales), over int8 / fp8 / int4 pages, on the MFMA (128),
+    many-column (96) and generic (72, int4 80) kernels; 4-D q and cu_seq_q; the output in half (bfloat16 too for int8 q)."""
     case = W.attn_case(torch.bfloat16, 140, kv=kv, B=5, Hq=8, Hkv=2, D=D, NB=64, max_ctx=150)
     q4 = _q_codes(qdt, (5, 2, 8, D), 141)
     qs4 = _q_scale(form, (5, 2, 8), 142, torch.bfloat16 if form == "token" else torch.float32)
@@ -692,12 +693,12 @@ def _sparse_tables(case, per, seed):
 
 
 @pytest.mark.parametrize("kv,D", [("int8_token", 128), ("int8_token", 96), ("plain", 128),
-                                  ("plain", 96), ("int4_token", 128)])
+                                  ("plain", 96), ("int4_token", 128), ("int8_token", 72), ("plain", 72)])
 @pytest.mark.parametrize("per", ["kv", "q"])
 def test_attn_sparse_tables(tmo, ref, dev, kv, per, D):
     """block_tables [batch, kv_heads or heads, max_blocks]: each KV head's (or query head's)
-    own pages; per-KV-head tables on the MFMA kernel, per-query-head tables with grouped heads
-    and head size 96 on the generic one; a missing page; 4-D q and cu_seq_q."""
+    own pages; per-KV-head tables on the MFMA (128) and many-column (96) kernels, per-query-head
+    tables with grouped heads and head size 72 on the generic one; a missing page; 4-D q and cu_seq_q."""
     case = W.attn_case(torch.bfloat16, 150, kv=kv, B=5, Hq=8, Hkv=2, D=D, NB=64, max_ctx=150)
     case.block_tables = _sparse_tables(case, 2 if per == "kv" else 8, 151)
     case.block_tables[2, 1, 1] = -1
@@ -889,8 +890,9 @@ def _many_columns(case, Hq, S, max_ctx):
 def test_attn_many_columns(tmo, ref, dev, kv, D, Hq, S, dtype, scales):
     """The many-column kernel over its kinds and head sizes: contexts at the edges of its 32- and
     64-key tiles, missing pages, a window, a sink, a negative softmax scale, ragged counts with
-    rows of no sequence, one split and several (an announced maximum of 12000 keys puts the whole
-    head sizes past the kernel's lower limit)."""
+    rows of no sequence, over several splits (an announced maximum of 12000 keys puts the whole
+    head sizes past the kernel's lower limit); with an unknown maximum these calls stay on the
+    other kernels, but for 80 and 96."""
     lens = [70, 1, 16, 64, 65, 127, 1500]
     case = W.attn_case(dtype, 160 + D, kv=kv, B=7, Hq=Hq, Hkv=2, D=D, BS=16, NB=700, max_ctx=1500,
                        scale_dtype=scales or torch.float32)
@@ -900,7 +902,8 @@ def test_attn_many_columns(tmo, ref, dev, kv, D, Hq, S, dtype, scales):
     q = W.attn_queries(dtype, 161, B=7, Hq=Hq, D=D, S=S)
     scale = D ** -0.5
     run_attn_mq(tmo, ref, dev, case, q, scale=scale, sink=torch.linspace(-1.0, 2.0, Hq), max_ctx=12000)
-    run_attn_mq(tmo, ref, dev, case, q, scale=-0.5 * scale, window=50, max_ctx=0)
+    for max_ctx in (0, 12000):
+        run_attn_mq(tmo, ref, dev, case, q, scale=-0.5 * scale, window=50, max_ctx=max_ctx)
     counts = [S, 1, min(16, S), 0, max(0, S - 3), min(3, S), S]
     q3, cu = W.attn_queries(dtype, 162, B=7, Hq=Hq, D=D, counts=counts)
     run_attn_mq(tmo, ref, dev, case, torch.cat([q3, q3[:2]]), cu=cu, scale=scale, max_seq_q=S,
