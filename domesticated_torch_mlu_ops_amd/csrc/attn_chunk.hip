@@ -99,7 +99,9 @@ struct Geo {
 
 // Workgroups per CU: two, and three where they fit (16-bit caches, head size 64: 191 us with two
 // for 8 chunks of up to 256 tokens over 8192 keys, 171 with three).
-template <int kD, int kKind, bool kQLo>
+// kFit: splits as long as the contexts present need (fitted_split).  That costs a workgroup's start
+// 0.5 to 1 us, so head sizes 80 and 96, whose calls had no faster kernel, keep the announced ones.
+template <int kD, int kKind, bool kQLo, bool kFit>
 __global__ __launch_bounds__(256, kD <= 64 && !chunk_quant(kKind) ? 3 : 2) void attn_chunk(AttnParams p) {
   using G = Geo<kD, kKind, kQLo>;
   constexpr bool kQuant = G::kQuant, kInt4 = G::kInt4;
@@ -110,6 +112,7 @@ __global__ __launch_bounds__(256, kD <= 64 && !chunk_quant(kKind) ? 3 : 2) void 
   __shared__ __align__(128) char lds_v[2][kT * kPitch];
   __shared__ __align__(16) float lds_ks[2][kT], lds_vs[2][kT];
 
+  touch_params();
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
@@ -117,16 +120,17 @@ __global__ __launch_bounds__(256, kD <= 64 && !chunk_quant(kKind) ? 3 : 2) void 
   // Longest sequences first, and of each the last column groups, which see the most keys: 707
   // -> 437 us for 8 chunks of up to 512 tokens over 1019..8192 int8 keys.  The KV heads of a
   // group are consecutive workgroups: with 8 of them, one per XCD and its L2.
-  const int64_t i = seq_by_length(p, (int)blockIdx.y);
+  const int32_t own = lane_length(p);
+  const int64_t i = seq_by_length(p, (int)blockIdx.y, own);
   const int hk = (int)(blockIdx.x % (unsigned)p.Hkv);
   const unsigned yr = (gridDim.x - 1 - blockIdx.x) / (unsigned)p.Hkv;
   const int cbg = (int)(yr / (unsigned)p.splits);  // group of 4 kC column blocks
   const int split = (int)yr - cbg * p.splits;
   const Seq sq = seq_of(p, i);
-  const int64_t per = fitted_split(p);
+  const int64_t per = kFit ? fitted_split(p, own) : p.split_tokens;
   const Range rg = token_range(p, sq, split, per);
   if (p.splits > 1 && rg.begin >= rg.end) return;  // an empty split writes no partial
-  const bool direct = live_splits(p, sq, per) <= 1;     // no merge: the only split writes the output
+  const bool direct = live_splits(p, sq, per) <= 1;  // no merge: the only split writes the output
 
   // the workgroup's keys: from its first token's window start to its last token's position
   constexpr int kCols = 64 * kC;
@@ -711,7 +715,10 @@ template <int kD, int kKind, bool kQLo>
 int launch_q(const AttnParams& p, hipStream_t st) {
   constexpr int kCols = 64 * Geo<kD, kKind, kQLo>::kC;
   const dim3 grid((unsigned)(p.Hkv * p.splits * ((p.ncols + kCols - 1) / kCols)), (unsigned)p.B);
-  return launch_kernel(attn_chunk<kD, kKind, kQLo>, grid, dim3(256), st, p);
+  if constexpr (kD % 64 == 0) {
+    if (p.few) return launch_kernel(attn_chunk<kD, kKind, kQLo, true>, grid, dim3(256), st, p);
+  }
+  return launch_kernel(attn_chunk<kD, kKind, kQLo, false>, grid, dim3(256), st, p);
 }
 
 template <int kD, int kKind>

@@ -67,13 +67,22 @@ struct AttnParams {
   int32_t splits;
   int32_t packed;                // 1-D grid, live workgroups first (work_of)
   int32_t lone;                  // a sequence's only live split writes the output itself
-  int32_t few;                   // many columns: splits that leave a CU at most one workgroup, or 0
+  int32_t few;                   // many columns: splits that leave a CU at most one workgroup, or 0: splits as announced
   int64_t split_tokens;          // multiple of 64 (latent caches: 32)
   float* ws;                     // [B, Hkv, splits, ncols, Dv + 2] when splits > 1
 };
 
 // ------------------------------------------------------------------------------ small helpers
 
+// One load from each 64-byte line of the launch parameters, together: the compiler loads them block
+// by block, and each first touch of a line is a round trip.
+__device__ __forceinline__ void touch_params() {
+  typedef const __attribute__((address_space(4))) uint32_t* Arg;
+  const Arg a = (Arg)__builtin_amdgcn_kernarg_segment_ptr();
+  constexpr int kLines = (sizeof(AttnParams) + 63) / 64;
+  static_assert(kLines == 8, "one load per line");
+  asm volatile("" ::"s"(a[0]), "s"(a[16]), "s"(a[32]), "s"(a[48]), "s"(a[64]), "s"(a[80]), "s"(a[96]), "s"(a[112]));
+}
 
 __device__ __forceinline__ uint16_t bf16_bits_rne(float x) {
   return __builtin_bit_cast(uint16_t, (__bf16)x);
@@ -150,13 +159,18 @@ __device__ __forceinline__ Seq seq_of(const AttnParams& p, int64_t i) {
   return q;
 }
 
+// Lane l: the length of sequence l (batches of up to 64; 0 past them and in larger ones), in one load.
+__device__ __forceinline__ int32_t lane_length(const AttnParams& p) {
+  const int lane = threadIdx.x & (kWave - 1);
+  return p.B <= kWave && lane < p.B ? p.lens[lane] : 0;
+}
+
 // The sequence of rank r by context length, longest first (batches of at most 64 sequences; r
 // itself in larger ones, which even out by their number).  Workgroups are dispatched in order, so
-// a long sequence that comes last would run on alone.
-__device__ __forceinline__ int64_t seq_by_length(const AttnParams& p, int r) {
+// a long sequence that comes last would run on alone.  own: lane_length.
+__device__ __forceinline__ int64_t seq_by_length(const AttnParams& p, int r, int32_t own) {
   if (p.B < 2 || p.B > kWave) return r;
   const int lane = threadIdx.x & (kWave - 1);
-  const int32_t own = lane < p.B ? p.lens[lane] : INT32_MIN;
   int rank = 0;
   for (int j = 0; j < p.B; ++j) {
     const int32_t other = __builtin_amdgcn_readlane(own, j);
@@ -190,13 +204,14 @@ __device__ __forceinline__ Range token_range(const AttnParams& p, const Seq& q, 
   return token_range(p, q, s, p.split_tokens);
 }
 
-// The many-column kernel's keys per split: as many as the split counts for the longest context
-// present would give, where the announced maximum (split_tokens) gives more.
-__device__ __forceinline__ int64_t fitted_split(const AttnParams& p) {
-  if (p.few < 2) return p.split_tokens;
-  uint32_t own = 0;
-  for (int j = threadIdx.x & (kWave - 1); j < p.B; j += kWave) own = max(own, (uint32_t)max(p.lens[j], 0));
-  const uint32_t longest = wave_max_u32_sgpr(own);
+// The many-column kernel's keys per split with p.few: as many as the split counts for the longest
+// context present would give, where the announced maximum (split_tokens) gives more.  own:
+// lane_length.
+__device__ __forceinline__ int64_t fitted_split(const AttnParams& p, int32_t own) {
+  uint32_t most = max(own, 0);
+  if (p.B > kWave)
+    for (int j = threadIdx.x & (kWave - 1); j < p.B; j += kWave) most = max(most, (uint32_t)max(p.lens[j], 0));
+  const uint32_t longest = wave_max_u32_sgpr(most);
   uint32_t n = (longest + 255) / 256;
   if (n > 1) n -= 1 - (n & 1);
   n = max(n, min((longest + 127) / 128, (uint32_t)p.few));

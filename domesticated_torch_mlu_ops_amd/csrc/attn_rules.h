@@ -27,11 +27,11 @@ namespace tmo {
 // us, 256 of 1 (128) 41 against 78, 256 of 8 (1024) 110 against 81; head size 256 (int4), 64 columns
 // of 8 and of 32 sequences 53 and 140 against 99 and 101.
 //
-// Codes of head size 64 are half the unpacking and MFMAs of 128, which attn_mfma hides better: they
-// need 112 columns and 2048 of its workgroups, whatever the splits.  8 KV heads, 2048 keys, 64
-// columns of 32 sequences int8 / float8 / int4 79 / 78 / 66 against 82 / 83 / 88 us; 256 columns of
-// 8 sequences, float8, 53 against 60 with one split and 71 against 53 with five, but 72 against 88
-// where the call announces 32768 keys; 256 columns of 32 sequences 200 against 140.
+// Codes of head size 64 are half the unpacking and MFMAs of 128, which attn_mfma hides better.  Half
+// empty workgroups lose: 8 KV heads, 2048 keys, 64 columns of 32 sequences int8 / float8 / int4 79 /
+// 78 / 66 against 82 / 83 / 88 us; 96 columns 112 / 109 / 90 against 83 / 83 / 92, 128 columns of 8
+// sequences 57 / 55 / 49 against 31 / 31 / 31.  One split needs more column blocks: 256 columns of 8
+// sequences (1024 workgroups of attn_mfma), float8, 53 against 60, 96 of 32 (1536) 87 against 62.
 inline bool attn_many_columns(bool codes, bool int4, int64_t head_size, int64_t cols, int64_t kv_heads,
                               int64_t batch, int64_t max_context_len, int64_t table_keys,
                               int64_t splits) {
@@ -40,7 +40,7 @@ inline bool attn_many_columns(bool codes, bool int4, int64_t head_size, int64_t 
   const int64_t keys = max_context_len > 0 ? max_context_len : table_keys;
   const int64_t blocks = (cols + 15) / 16, all = blocks * kv_heads * batch;
   if (blocks < 4 || (double)cols * (double)kv_heads * (double)batch * (double)keys <= 5e6) return false;
-  if (codes && head_size == 64) return blocks >= 7 && all >= 2048;
+  if (codes && head_size == 64) return blocks >= (int4 ? 7 : 6) && (splits > 1 || all >= 1536);
   return splits > 1 || all >= 1024;
 }
 

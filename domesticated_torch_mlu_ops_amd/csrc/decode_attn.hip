@@ -47,7 +47,7 @@ __global__ __launch_bounds__(256) void attn_combine(AttnParams p) {
   const int64_t stride = (int64_t)p.ncols * (p.Dv + 2);
   const float* base = p.ws + ((i * p.Hkv + hk) * p.splits * (int64_t)p.ncols + c) * (p.Dv + 2);
   // splits past the sequence's keys wrote nothing (the main kernel returned early)
-  const int live = live_splits(p, sq, p.lone ? fitted_split(p) : p.split_tokens);
+  const int live = live_splits(p, sq, p.few ? fitted_split(p, lane_length(p)) : p.split_tokens);
   if (p.lone && live == 1) return;
   // Every load is unconditional (split and channel indices clamped into this column's rows of
   // the workspace; an empty split's row is read and given weight 0), so the loads of a batch
@@ -591,7 +591,14 @@ extern "C" int tmo_hip_cached_kv_attn(
   if (chunk) {
     p.lone = 1;
     p.packed = 0;
-    p.few = p.splits > 1 ? (int32_t)(255 / (batch * num_kv_heads * ((p.ncols + 127) / 128))) : 0;
+    // Splits as long as the contexts present need where the announced ones could make the call
+    // slower than on attn_mfma: whole head sizes with fewer than 128 workgroups per split (256 for
+    // codes of 64).  64 columns of 8 sequences of 2048 int8 keys, head size
+    // 128, announced as 32768: 76 us on attn_mfma, 88 with the announced splits, 46 with fitted ones.
+    if (whole && p.splits > 1) {
+      p.few = (int32_t)(255 / (batch * num_kv_heads * ((p.ncols + 127) / 128)));
+      if (p.few == 1 && !(quant && head_size == 64)) p.few = 0;
+    }
     const int rc = launch_attn_chunk(p, qlo, st);
     return rc != TMO_OK || p.splits == 1 ? rc : launch_combine(p, st);
   }

@@ -865,7 +865,7 @@ def _many_columns(case, Hq, S, max_ctx):
     if blocks < 4 or cols * seqs * keys <= 5e6:
         return False
     if D == 64 and case.k_scale is not None:
-        return blocks >= 7 and blocks * seqs >= 2048
+        return blocks >= (7 if case.int4 else 6) and (max_ctx > 256 or blocks * seqs >= 1536)
     return max_ctx > 256 or blocks * seqs >= 1024
 
 
