@@ -24,7 +24,7 @@
 //     side by side; V^T takes the same token order.
 //   * p enters as hi + lo operands of 16 significant bits, as in attn_mfma.
 // 32 sequences of 512..8192 rows, 16 heads, bf16 (157 MB): 34.3 ms on the VALU kernel that served
-// this form before, 45 us here (3.5 TB/s), of which 6 are the merging of the splits.  One
+// this form before, 45 us here (3.5 TB/s), of which 7.5 are the merging of the splits.  One
 // workgroup alone takes 1.33 us per 32-row tile; two per CU cover each other's latencies, and
 // what is left is their uneven share of ragged contexts.
 #include "attn_common.h"
