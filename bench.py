@@ -68,8 +68,8 @@ KERNELS = {"cfg1": "quant_paged_vec<BF16,16,1,false>", "cfg2": "quant_paged_vec<
            "fused_rope_ln": "fused_rope_tok<BF16,16,3,1,256>",
            "fused_rope_70b": "fused_rope_tok<BF16,16,3,0,512>",
            "linear_quant": "lin_quant<BF16,16,false,false,true>", "linear_dequant": "lin_dequant<BF16,16>",
-           "linear_reshape": "lin_copy<16,true>", "decode_attn": "attn_mfma<128,0,false,false,false>",
-           "reshape_paged": "reshape_paged_rows<16>", "decode_attn_int4": "attn_mfma<128,4,false,false,false>"}
+           "linear_reshape": "lin_copy<16,true>", "decode_attn": "attn_mfma<128,0,false,false,false,true>",
+           "reshape_paged": "reshape_paged_rows<16>", "decode_attn_int4": "attn_mfma<128,4,false,false,false,true>"}
 
 
 def parse_args():
